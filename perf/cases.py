@@ -320,7 +320,7 @@ def tolerance(case):
     if case["kind"] != "block":
         return {"rel": 1e-5, "max": 1e-3}
     # Through the projection a code next to an edge may fall to its other side (see the top);
-    # at 512 cached positions or more one such code moves an attention output by a part in a
+    # at 250 cached positions or more one such code moves an attention output by a part in a
     # few hundred at most.  (The projections themselves: seen up to 5e-7 off 64 bits.)
     return {"rel": 1e-3, "max": 0.2}
 
