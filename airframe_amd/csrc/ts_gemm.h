@@ -8,6 +8,8 @@
 // chunk are 64 contiguous bytes of its weight row.  D register 4q + r of a 32 x 32 block is
 // row 8q + 4hf + r, column j.
 #pragma once
+#include <type_traits>
+
 #include "ts_mfma.h"
 
 namespace ts {
@@ -34,89 +36,168 @@ __device__ inline void zero(floatx16 &a) {
     for (int e = 0; e < 16; e++) a[e] = 0.0f;
 }
 
-// x tiles of MT rows, double-buffered, for the tile loop.
-template <int MT>
-struct XTiles {
-    _Float16 hi[2][MT][kAStr];
-    _Float16 lo[2][MT][kAStr];
+// LDS of the tile loop: three chunks of kTK k of 64 x rows (hi/lo) and 256 weight rows, rows
+// unpadded.  A row's four 16-byte slots are permuted by row (tile_slot) so that the 16 rows
+// that one phase of an operand read or a staging write touches at one slot cover all 64 banks.
+constexpr int kTK = 32;
+struct GemmTiles {
+    _Float16 hi[3][64][kTK];
+    _Float16 lo[3][64][kTK];
+    _Float16 w[3][256][kTK];
 };
+// f16 index inside tile row r of slot s (8 k).
+__device__ inline int tile_slot(int r, int s) { return 8 * (s ^ ((r >> 2) & 3)); }
 
-// MT = 64 WR rows x 256 columns over nch chunks, 256 WR threads: wave (wr, wc) accumulates rows
-// 64 wr + 32 rb + .., columns 64 wc + 32 cb + .. in acc[rb][cb].  Staging thread (si = tid / 4,
-// sc = tid % 4) owns 16 floats of x row si per chunk: xs points at them for chunk 0 (null: a
-// zero row).  wp[cb]: the lane's weight row of column block cb at its chunk-0 offset 32 hf.
-// xwrap: x has xwrap chunks and weight chunk c multiplies x chunk c mod xwrap (nch = 2 xwrap:
-// rows of two weight planes, hi then lo, against the same x; nch = xwrap: one plane).
-// Both operands run D chunks ahead: x and the weights of chunk c + D are loaded into a ring of
-// D register sets while chunk c is multiplied, and x of chunk c + 1 goes to LDS (hi/lo,
-// double-buffered) after chunk c's matrix work, so each load has D - 1 iterations to arrive.
-// D = 3 keeps two waves per SIMD; measured 10% faster than x one chunk and the weights two
-// chunks ahead, while D = 4 drops to one wave per SIMD and is slower.
-template <int WR, int D = 3>
-__device__ __forceinline__ void gemm_tile_core(XTiles<64 * WR> &sm, const float *xs,
-                                                    const _Float16 *const (&wp)[2], int nch, int xwrap,
-                                                    int tid, floatx16 (&acc)[2][2]) {
-    const int wave = tid >> 6, lane = tid & 63, j = lane & 31, hf = lane >> 5, wr = wave >> 2;
+#define TS_SGB(mask, n) __builtin_amdgcn_sched_group_barrier(mask, n, 0)
+constexpr int kValu = 2, kMfma = 8, kVmemRead = 0x20, kDsRead = 0x100, kDsWrite = 0x200;
+
+// 64 rows x 256 columns over nch chunks of kTK, 256 threads: wave w accumulates rows 32 rb + ..,
+// columns 64 w + 32 cb + .. in acc[rb][cb].  Staging thread tid owns slot tid % 4 of x row tid / 4
+// and of weight rows tid / 4 + 64 i: xs / ws[i] point at it in chunk 0 (a row past the tile's last
+// one points at any valid row: what it adds up to is not used).  xwrap: x has xwrap chunks and
+// weight chunk c multiplies x chunk c mod xwrap (nch = 2 xwrap: rows of two weight planes, hi
+// then lo, against the same x; nch = xwrap: one plane).
+//
+// Both operands go through LDS, read from memory whole cache lines at a time (a weight row per
+// lane, straight into the operands, kept the address path busier than the matrix cores).  Chunk c
+// is multiplied from one LDS buffer while chunk c + 2 goes from registers into another and
+// chunk c + 5 is loaded into those registers; the third buffer already holds chunk c + 1, so that
+// its first operands are read before the barrier and no matrix instruction waits for LDS
+// behind it.  The instruction groups spread the staging's VALU, LDS and memory instructions
+// between the matrix instructions of the same wave (two waves per SIMD do not cover for each
+// other between barriers).  Nothing in the loop is conditional (a skipped load would make every
+// wait for memory a wait for all of it): past the end the last chunk is loaded and stored again.
+// 2048 x 6144 outputs, 2560 long: 198 us with the weight rows loaded into the operands, 164 now
+// (785 TFLOP/s executed; all CUs together reach about 1.1 PFLOP/s on f16 matrix instructions).
+// LDS bounds it: per chunk 48 KB read at 128 and 24 KB written at 75 bytes a clock, ~710 clocks
+// against 512 of matrix work.  128-row tiles (8 waves, or 4 of 64 x 128) were slower.
+__device__ __forceinline__ void gemm_tile_core(GemmTiles &sm, const float *xs, const _Float16 *const (&ws)[4],
+                                               int nch, int xwrap, int tid, floatx16 (&acc)[2][2]) {
+    const int wave = tid >> 6, lane = tid & 63, j = lane & 31, hf = lane >> 5;
     const int si = tid >> 2, sc = tid & 3;
+    struct Stage {
+        float4 x[2];
+        half8 w[4];
+    };
+    struct Ops {
+        half8 ah[2], al[2], b[2];
+    };
+    auto load = [&](Stage &g, int c) {
+        c = min(c, nch - 1);
+        const int cx = c >= xwrap ? c - xwrap : c;
+        g.x[0] = *reinterpret_cast<const float4 *>(xs + (size_t)cx * kTK);
+        g.x[1] = *reinterpret_cast<const float4 *>(xs + (size_t)cx * kTK + 4);
+#pragma unroll
+        for (int i = 0; i < 4; i++) g.w[i] = *reinterpret_cast<const half8 *>(ws[i] + (size_t)c * kTK);
+    };
+    auto store_x = [&](int buf, const Stage &g) {
+        const int at = tile_slot(si, sc);
+        half8 h, l;
+        split8(g.x[0], g.x[1], h, l);
+        *reinterpret_cast<half8 *>(&sm.hi[buf][si][at]) = h;
+        *reinterpret_cast<half8 *>(&sm.lo[buf][si][at]) = l;
+    };
+    auto store_w = [&](int buf, const Stage &g) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int r = si + 64 * i;
+            *reinterpret_cast<half8 *>(&sm.w[buf][r][tile_slot(r, sc)]) = g.w[i];
+        }
+    };
+    auto fetch = [&](Ops &o, int buf, int q) {
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++) {
+            const int r = 32 * rb + j, at = tile_slot(r, 2 * q + hf);
+            o.ah[rb] = *reinterpret_cast<const half8 *>(&sm.hi[buf][r][at]);
+            o.al[rb] = *reinterpret_cast<const half8 *>(&sm.lo[buf][r][at]);
+        }
+#pragma unroll
+        for (int cb = 0; cb < 2; cb++) {
+            const int r = 64 * wave + 32 * cb + j;
+            o.b[cb] = *reinterpret_cast<const half8 *>(&sm.w[buf][r][tile_slot(r, 2 * q + hf)]);
+        }
+    };
+    auto multiply = [&](const Ops &o) {
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++)
+#pragma unroll
+            for (int cb = 0; cb < 2; cb++)
+                acc[rb][cb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(o.ah[rb], o.b[cb], acc[rb][cb], 0, 0, 0);
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++)
+#pragma unroll
+            for (int cb = 0; cb < 2; cb++)
+                acc[rb][cb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(o.al[rb], o.b[cb], acc[rb][cb], 0, 0, 0);
+    };
 #pragma unroll
     for (int rb = 0; rb < 2; rb++)
 #pragma unroll
         for (int cb = 0; cb < 2; cb++) zero(acc[rb][cb]);
-
-    float4 xq[D][4];
-    half8 wq[D][2][4];
-    auto load = [&](float4 (&x)[4], half8 (&w)[2][4], int c) {
-        const bool on = c < nch;
-        const int cx = c >= xwrap ? c - xwrap : c;
+    Stage g[3];
+    Ops o[2];
 #pragma unroll
-        for (int u = 0; u < 4; u++)
-            x[u] = (xs && on) ? *reinterpret_cast<const float4 *>(xs + cx * kKC + 4 * u) : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int u = 0; u < 3; u++) load(g[u], u);
 #pragma unroll
-        for (int cb = 0; cb < 2; cb++)
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-                w[cb][q] = on ? *reinterpret_cast<const half8 *>(wp[cb] + c * kKC + 8 * q) : (half8)(_Float16)0.0f;
-    };
-    auto store_x = [&](int buf, const float4 (&x)[4]) {
-        half8 h, l;
-        split8(x[0], x[1], h, l);
-        *reinterpret_cast<half8 *>(&sm.hi[buf][si][16 * sc]) = h;
-        *reinterpret_cast<half8 *>(&sm.lo[buf][si][16 * sc]) = l;
-        split8(x[2], x[3], h, l);
-        *reinterpret_cast<half8 *>(&sm.hi[buf][si][16 * sc + 8]) = h;
-        *reinterpret_cast<half8 *>(&sm.lo[buf][si][16 * sc + 8]) = l;
-    };
-#pragma unroll
-    for (int u = 0; u < D; u++) load(xq[u], wq[u], u);
-    store_x(0, xq[0]);
-    __syncthreads();
-
-    for (int c0 = 0; c0 < nch; c0 += D) {
-#pragma unroll
-        for (int u = 0; u < D; u++) {
-            const int c = c0 + u;
-            if (c < nch) {  // uniform
-                const int buf = c & 1;
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-#pragma unroll
-                    for (int rb = 0; rb < 2; rb++) {
-                        const int row = 64 * wr + 32 * rb + j;
-                        const half8 ah = *reinterpret_cast<const half8 *>(&sm.hi[buf][row][32 * hf + 8 * q]);
-                        const half8 al = *reinterpret_cast<const half8 *>(&sm.lo[buf][row][32 * hf + 8 * q]);
-#pragma unroll
-                        for (int cb = 0; cb < 2; cb++) {
-                            acc[rb][cb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, wq[u][cb][q], acc[rb][cb], 0, 0, 0);
-                            acc[rb][cb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, wq[u][cb][q], acc[rb][cb], 0, 0, 0);
-                        }
-                    }
-                }
-                if (c + 1 < nch) store_x(buf ^ 1, xq[(u + 1) % D]);
-                load(xq[u], wq[u], c + D);
-                __syncthreads();
-            }
-        }
+    for (int u = 0; u < 2; u++) {
+        store_x(u, g[u]);
+        store_w(u, g[u]);
+        load(g[u], 3 + u);
     }
+    __syncthreads();
+    fetch(o[0], 0, 0);
+    // chunk c in buffer u = c mod 3 (a constant, so that g and o stay in registers)
+    auto step = [&](auto uc, int c) {
+        constexpr int u = decltype(uc)::value, v = (u + 2) % 3;
+        fetch(o[1], u, 1);
+        store_x(v, g[v]);
+        multiply(o[0]);
+#pragma unroll
+        for (int i = 0; i < 6; i++) {
+            TS_SGB(kMfma, 1);
+            TS_SGB(kDsRead, 1);
+            TS_SGB(kValu, 5);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            TS_SGB(kMfma, 1);
+            TS_SGB(kValu, 6);
+            TS_SGB(kDsWrite, 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(o[0], (u + 1) % 3, 0);
+        store_w(v, g[v]);
+        load(g[v], c + 5);
+        multiply(o[1]);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            TS_SGB(kMfma, 1);
+            TS_SGB(kDsRead, 1);
+            TS_SGB(kDsWrite, 1);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            TS_SGB(kMfma, 1);
+            TS_SGB(kDsRead, 1);
+            TS_SGB(kValu, 4);
+            TS_SGB(kVmemRead, 1);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            TS_SGB(kMfma, 1);
+            TS_SGB(kValu, 4);
+            TS_SGB(kVmemRead, 2);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+    };
+    int c = 0;
+    for (; c + 3 <= nch; c += 3) {
+        step(std::integral_constant<int, 0>{}, c);
+        step(std::integral_constant<int, 1>{}, c + 1);
+        step(std::integral_constant<int, 2>{}, c + 2);
+    }
+    if (c < nch) step(std::integral_constant<int, 0>{}, c);
+    if (c + 1 < nch) step(std::integral_constant<int, 1>{}, c + 1);
 }
 
 // LDS of gemm_split_core: x of one batch (4 chunks) as hi/lo.

@@ -44,34 +44,42 @@ __device__ inline void proj_tile_of(const ProjArgs &p, int id, int &rt, int &ct,
     sp = lin / (p.RT * p.CT);
 }
 
-__device__ inline void proj_out(const ProjArgs &p, int row, int col, float v) {
-    if (row >= p.M || col >= p.N) return;
-    const size_t i = (size_t)row * p.N + col;
-    if (p.stash) p.stash[i] = v;
-    p.act[i] = p.act[i] + v;
-}
-
-// 64-row tiles over all of K; the epilogue from the accumulators.
-__global__ __launch_bounds__(256) void proj_tile_kernel(ProjArgs p) {
-    __shared__ __align__(16) XTiles<64> sm;
+// 64-row tiles over all of K; the epilogue from the accumulators.  The residuals of a 32 x 32
+// block are loaded together before any of them is used (one by one, each a trip to memory, they
+// took as long as the whole product of a 96-long reduction: 51 us of 2048 x 6144 outputs).
+__global__ __launch_bounds__(256, 2) void proj_tile_kernel(ProjArgs p) {
+    __shared__ __align__(16) GemmTiles sm;
     int rt, ct, sp;
     proj_tile_of(p, blockIdx.x, rt, ct, sp);
     if (sp >= 1) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 31, hf = lane >> 5;
-    const int row0 = 64 * rt, col0 = kPT * ct + 64 * wave;
+    const int row0 = 64 * rt, col0 = kPT * ct;
     const int si = tid >> 2, sc = tid & 3;
-    const float *xs = row0 + si < p.M ? p.a + (size_t)(row0 + si) * p.K + 16 * sc : nullptr;
-    const _Float16 *const wp[2] = {p.w + (size_t)min(col0 + j, p.N - 1) * p.KW + 32 * hf,
-                                   p.w + (size_t)min(col0 + 32 + j, p.N - 1) * p.KW + 32 * hf};
+    const float *xs = p.a + (size_t)min(row0 + si, p.M - 1) * p.K + 8 * sc;
+    const _Float16 *ws[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) ws[i] = p.w + (size_t)min(col0 + si + 64 * i, p.N - 1) * p.KW + 8 * sc;
     floatx16 acc[2][2];
-    gemm_tile_core<1>(sm, xs, wp, p.KW / kKC, p.K / kKC, tid, acc);
+    gemm_tile_core(sm, xs, ws, p.KW / kTK, p.K / kTK, tid, acc);
 #pragma unroll
     for (int rb = 0; rb < 2; rb++)
 #pragma unroll
-        for (int cb = 0; cb < 2; cb++)
+        for (int cb = 0; cb < 2; cb++) {
+            const int col = col0 + 64 * wave + 32 * cb + j;
+            const int r0 = row0 + 32 * rb + 4 * hf;
+            float res[16];
 #pragma unroll
             for (int e = 0; e < 16; e++)
-                proj_out(p, row0 + 32 * rb + 8 * (e >> 2) + 4 * hf + (e & 3), col0 + 32 * cb + j, acc[rb][cb][e]);
+                res[e] = p.act[(size_t)min(r0 + 8 * (e >> 2) + (e & 3), p.M - 1) * p.N + min(col, p.N - 1)];
+#pragma unroll
+            for (int e = 0; e < 16; e++) {
+                const int row = r0 + 8 * (e >> 2) + (e & 3);
+                if (row >= p.M || col >= p.N) continue;
+                const size_t i = (size_t)row * p.N + col;
+                if (p.stash) p.stash[i] = acc[rb][cb][e];
+                p.act[i] = res[e] + acc[rb][cb][e];
+            }
+        }
 }
 
 // One split of the reduction on a 32-row tile; the partial to the scratch buffer.

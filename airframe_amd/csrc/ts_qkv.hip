@@ -25,8 +25,6 @@
 //   * Few tiles (decode): 32-row tiles with the reduction over dim split across workgroups
 //     (gemm_split_core, one memory round trip per slice), f32 partials, and a second kernel
 //     that sums them in split order (deterministic) and runs the epilogue.
-#include <type_traits>
-
 #include "ts_gemm.h"
 #include "ts_kquant.h"
 #include "ts_store.h"
@@ -38,11 +36,6 @@ constexpr int kMT = 32;     // rows per tile
 constexpr int kNT = 256;    // columns per tile
 constexpr int kTStr = 260;  // LDS row stride of the output tile (f32)
 constexpr int kMaxSplit = 16;  // most splits of the reduction over dim
-// V blocks per row tile of the prefill kernel: 64 rows.  (128 rows, two row waves per column
-// of waves, measured 270 vs 190 us on the config-5 shape: the row waves each load the same
-// weights, so the larger tile only adds registers.)
-constexpr int kBigBlocks = 2;
-
 
 struct QkvArgs {
     KvLayerView L;
@@ -285,76 +278,129 @@ __device__ void qkv_epilogue(const QkvArgs &a, const RowTile &t, int ct, const f
         store_kv_tile<64>(a, t, ct, tile, r0, nr, tid);
 }
 
-// One workgroup per tile over all of dim (grids with enough tiles): MT = 64 WR rows -- for
-// block rows 2 WR consecutive V blocks of one sequence, for decode rows MT sequences -- through
-// gemm_tile_core (each wave 64 x 64, 2 x 2 MFMA blocks: every weight operand feeds two row
-// blocks and every x operand two column blocks).  The epilogue runs 32 rows at a time on a
-// 32 x 256 LDS tile that reuses the x buffers.
-template <int WR>
-__global__ __launch_bounds__(256 * WR) void qkv_tile_kernel(QkvArgs a) {
-    constexpr int MT = 64 * WR, NBLK = MT / kBlk;
+// Row units u0 .. u0 + N - 1 of a prefill call: unit u is the u-th live V block, sequence by
+// sequence (sequence s has live blocks len[s] / 32 .. (end - 1) / 32), so that a tile's 32-row
+// units may come from several sequences and no tile is spent on blocks that a sequence's
+// start leaves empty.  64 sequences at a time, one per lane.
+// Called by one wave.
+template <int N>
+__device__ inline void find_units(const QkvArgs &a, int u0, RowTile (&t)[N]) {
+    const int lane = threadIdx.x & 63;
+    if (lane < N) t[lane].live = false;
+    int before = 0;  // units of the sequences before `base`
+    for (int base = 0; base < a.L.S && before < u0 + N; base += 64) {
+        const int s = base + lane;
+        const int start = s < a.L.S ? a.len[s] : 0;
+        const int end = min(start + a.n_tok, a.L.P);
+        const int n = s < a.L.S && end > start ? (end - 1) / kBlk - start / kBlk + 1 : 0;
+        int upto = n;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(upto, d, 64);
+            if (lane >= d) upto += o;
+        }
+        const int first = before + upto - n;  // the first unit of sequence s
+        for (int i = 0; i < N; i++) {
+            const int k = u0 + i - first;
+            if (k < 0 || k >= n) continue;
+            const int blk = start / kBlk + k;
+            t[i].s = s;
+            t[i].start = start;
+            t[i].blk = blk;
+            t[i].lo = max(blk * kBlk, start);
+            t[i].hi = min(blk * kBlk + kBlk, end);
+            t[i].live = true;
+        }
+        before += __shfl(upto, 63, 64);
+    }
+}
+
+// One workgroup per tile over all of dim (grids with enough tiles): 64 rows -- for block rows two
+// live V blocks (find_units), for decode rows 64 sequences -- through gemm_tile_core (each wave
+// 64 x 64, 2 x 2 MFMA blocks: every weight operand feeds two row blocks and every x operand two
+// column blocks).  q goes out straight from the accumulators; for K and V the epilogue runs 32
+// rows at a time on a 32 x 256 LDS tile that reuses the operand buffers.
+__global__ __launch_bounds__(256, 2) void qkv_tile_kernel(QkvArgs a) {
+    constexpr int MT = 64, NU = MT / kMT;
     union Smem {
-        XTiles<MT> x;
+        GemmTiles x;
         float tile[kMT][kTStr];
     };
     __shared__ __align__(16) Smem sm;
+    __shared__ RowTile t[NU];
 
     int rt, ct, sp;
     tile_of(a, blockIdx.x, rt, ct, sp);
     if (sp >= a.n_split) return;
-    const bool single = a.n_tok == 1;  // decode rows: MT sequences, one token each
-    const int nb4 = (a.n_tok / kBlk + 2 + NBLK - 1) / NBLK;
-    const int s = single ? MT * rt : rt / nb4;
-    const int start = single ? 0 : a.len[s], end = single ? a.n_tok : min(start + a.n_tok, a.L.P);
-    const int blk0 = start / kBlk + NBLK * (rt % nb4);
-    if (!single && blk0 * kBlk >= end) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 31, hf = lane >> 5;
-    const int wr = wave >> 2, wc = wave & 3;
+    if (a.n_tok == 1) {
+        if (tid < NU) {
+            RowTile u;
+            u.s = MT * rt + kMT * tid;
+            u.blk = u.start = u.lo = u.hi = 0;
+            u.live = u.s < a.L.S;
+            t[tid] = u;
+        }
+    } else if (wave == 0) {
+        find_units(a, NU * rt, t);
+    }
+    __syncthreads();
+    if (!t[0].live) return;  // (units are live from the first one on)
 
-    // staging role: row si (0..MT-1), 16 floats at k offset 16 sc of each chunk
+    // staging roles: x row si (an empty row reads the first unit's first live one)
     const int si = tid >> 2, sc = tid & 3;
-    const int ps = blk0 * kBlk + si;
-    const int xr = single ? (s + si < a.L.S ? s + si : -1)
-                          : (ps >= start && ps < end) ? s * a.n_tok + (ps - start) : -1;
-    const float *xs = xr >= 0 ? a.x + (size_t)xr * a.dim + 16 * sc : nullptr;
-    const _Float16 *const wp[2] = {w_row(a, ct, 64 * wc + j) + 32 * hf, w_row(a, ct, 64 * wc + 32 + j) + 32 * hf};
+    const RowTile us = t[si / kMT];
+    int xr = us.live ? x_row(a, us, si % kMT) : -1;
+    if (xr < 0) xr = x_row(a, t[0], a.n_tok == 1 ? 0 : t[0].lo - t[0].blk * kBlk);
+    const float *xs = a.x + (size_t)xr * a.dim + 8 * sc;
+    const _Float16 *ws[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) ws[i] = w_row(a, ct, si + 64 * i) + 8 * sc;
     floatx16 acc[2][2];
-    gemm_tile_core<WR>(sm.x, xs, wp, a.wld / kKC, a.dim / kKC, tid, acc);
+    gemm_tile_core(sm.x, xs, ws, a.wld / kTK, a.dim / kTK, tid, acc);
 
-    // Epilogue, one 32-row block at a time: the waves holding it (wr = b / 2, row block b % 2)
-    // write it to the LDS tile, then the first 4 waves run the block's epilogue.  The block
-    // index is a template constant so that acc is indexed with constants and stays in
-    // registers.
+    if (ct < a.n_qt) {
+        const int ld = a.n_head * a.hd;
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            // live rows [lo, hi) of the unit, row 0 at x row r0
+            const RowTile u = t[b];
+            const bool single = a.n_tok == 1;
+            const int p0 = u.blk * kBlk;
+            const int lo = single ? 0 : u.lo - p0;
+            const int hi = !u.live ? lo : single ? min(kMT, a.L.S - u.s) : u.hi - p0;
+            const int64_t r0 = single ? u.s : (int64_t)u.s * a.n_tok + (p0 - u.start);
+#pragma unroll
+            for (int cb = 0; cb < 2; cb++) {
+                const int col = ct * kNT + 64 * wave + 32 * cb + j;
+                if (col >= ld) continue;
+                float *dst = a.q_out + (r0 + 4 * hf) * ld + col;
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    const int i = 8 * (e >> 2) + (e & 3);
+                    if ((unsigned)(i + 4 * hf - lo) < (unsigned)(hi - lo)) dst[(size_t)i * ld] = acc[b][cb][e];
+                }
+            }
+        }
+        return;
+    }
+    // (the block index is a template constant, so that acc is indexed with constants and stays in
+    // registers)
     auto block = [&](auto bc) {
         constexpr int b = decltype(bc)::value;
-        if constexpr (b < NBLK) {
-            const int p0 = (blk0 + b) * kBlk;
-            if (single ? s + kBlk * b >= a.L.S : p0 >= end) return;  // uniform
-            if (wr == (b >> 1)) {
+        const RowTile u = t[b];
+        if (!u.live) return;  // uniform
 #pragma unroll
-                for (int cb = 0; cb < 2; cb++)
+        for (int cb = 0; cb < 2; cb++)
 #pragma unroll
-                    for (int e = 0; e < 16; e++)
-                        sm.tile[8 * (e >> 2) + 4 * hf + (e & 3)][64 * wc + 32 * cb + j] = acc[b & 1][cb][e];
-            }
-            __syncthreads();
-            if (tid < 256) {
-                RowTile t;
-                t.s = single ? s + kBlk * b : s;
-                t.start = start;
-                t.blk = blk0 + b;
-                t.lo = max(p0, start);
-                t.hi = min(p0 + kBlk, end);
-                t.live = true;
-                qkv_epilogue(a, t, ct, sm.tile, 0, kMT, tid);
-            }
-            __syncthreads();
-        }
+            for (int e = 0; e < 16; e++)
+                sm.tile[8 * (e >> 2) + 4 * hf + (e & 3)][64 * wave + 32 * cb + j] = acc[b][cb][e];
+        __syncthreads();
+        qkv_epilogue(a, u, ct, sm.tile, 0, kMT, tid);
+        __syncthreads();
     };
     block(std::integral_constant<int, 0>{});
     block(std::integral_constant<int, 1>{});
-    block(std::integral_constant<int, 2>{});
-    block(std::integral_constant<int, 3>{});
 }
 
 // One split of the reduction for small grids (decode) through gemm_split_core; the f32
@@ -461,10 +507,9 @@ QkvPlan qkv_plan(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok) {
         p.part_bytes = (uint64_t)p.n_split * tiles * kMT * kNT * sizeof(float);
         return p;
     }
-    // Otherwise one workgroup per tile of 32 kBigBlocks rows over all of dim.
+    // Otherwise one workgroup per tile of two 32-row units over all of dim.
     p.big = true;
-    const int mt = kBlk * kBigBlocks;
-    p.RT = n_tok == 1 ? (n_seq + mt - 1) / mt : n_seq * ((n_tok / kBlk + 2 + kBigBlocks - 1) / kBigBlocks);
+    p.RT = (rt32 + 1) / 2;
     return p;
 }
 
@@ -571,7 +616,7 @@ hipError_t launch_qkv(const KvLayerView &L, const int32_t *d_len, const float *x
     a.n_wg = plan.RT * plan.CT * plan.n_split;
     const int grid = (a.n_wg + 7) / 8 * 8;
     if (plan.big) {
-        qkv_tile_kernel<kBigBlocks / 2><<<grid, 128 * kBigBlocks, 0, st>>>(a);
+        qkv_tile_kernel<<<grid, 256, 0, st>>>(a);
     } else {
         qkv_split_kernel<<<grid, 256, 0, st>>>(a);
         if (n_tok == 1)
