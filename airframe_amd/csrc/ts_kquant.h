@@ -1,6 +1,6 @@
 // ts_kquant.h -- projection weights in the GGUF block formats Q4_K, Q5_K (below) and Q8_0,
-// Q4_0 (further down) read at their own size inside the matrix-core loop of the split
-// projections (decode shapes).
+// Q4_0 (further down) read at their own size inside the matrix-core loops of the projections:
+// slices of the reduction for few rows, and 64-row tiles over all of it for many (at the end).
 //
 // The reference's main_qkv / main_attn_proj read every weight from the GGUF blob inside the dot
 // product (src/backend/bindless/sh_layer_v1_int4.wgsl:502-520, sh_layer_v1.wgsl:777-790) with
@@ -40,6 +40,28 @@ struct KQ {
 __host__ __device__ constexpr bool kq_type(int t) {
     return t == kGgmlQ4_0 || t == kGgmlQ5_0 || t == kGgmlQ8_0 || t == kGgmlQ4K || t == kGgmlQ5K;
 }
+
+// f(integral_constant<int, type>) for a block type known at run time.
+template <typename F>
+void kq_dispatch(int t, F f) {
+    if (t == kGgmlQ4K)
+        f(std::integral_constant<int, kGgmlQ4K>{});
+    else if (t == kGgmlQ5K)
+        f(std::integral_constant<int, kGgmlQ5K>{});
+    else if (t == kGgmlQ8_0)
+        f(std::integral_constant<int, kGgmlQ8_0>{});
+    else if (t == kGgmlQ5_0)
+        f(std::integral_constant<int, kGgmlQ5_0>{});
+    else
+        f(std::integral_constant<int, kGgmlQ4_0>{});
+}
+// Whether a projection of that many 32 x 256 tiles takes the 64-row tile loop over the whole
+// reduction (one round of half as many workgroups) instead of slices and partials.  Measured
+// either way on whole blocks of 100 to 600 tokens, 2048 to 4096 wide: Q4_K, Q5_K and Q4_0 lose
+// 0.78-0.99 of their speed below 256 tiles and gain 1.06-1.27 just above (300 tokens of 4096: 1.06,
+// 420 of 3072: 1.27); Q8_0 and Q5_0, whose slices decode more, gain 1.05-1.2 from 192 tiles on
+// and lose below 160.
+inline bool kq_tiles(int t, int tiles32) { return tiles32 >= (t == kGgmlQ8_0 || t == kGgmlQ5_0 ? 192 : 256); }
 
 // LDS of the K-quant slice loop: x of one super-block (4 chunks of 64) as hi/lo, and the f32
 // sums of its 8 sub-blocks per row.
@@ -282,24 +304,41 @@ struct QbRegs {
     uint32_t y[4];  // Q5_0: even block 2k: its sixth dword
 };
 
-template <int T>
-__device__ __forceinline__ void qb_load(QbRegs &r, const uint8_t *sb, int hf) {
+// A T at p, in p's address space.
+typedef const __attribute__((address_space(1))) uint8_t *global_bytes;
+template <typename T>
+__device__ inline T load_as(const uint8_t *p) {
+    return *reinterpret_cast<const T *>(p);
+}
+template <typename T>
+__device__ inline T load_as(global_bytes p) {
+    return *reinterpret_cast<const __attribute__((address_space(1))) T *>(p);
+}
+
+// Blocks 2k and 2k + 1.
+template <int T, typename P>
+__device__ __forceinline__ void qb_load_pair(QbRegs &r, P sb, int hf, int k) {
     typedef uint32_t u32x4a __attribute__((ext_vector_type(4), aligned(4)));
     constexpr int BB = T == kGgmlQ8_0 ? 34 : T == kGgmlQ5_0 ? 22 : 18;
     const int off = T == kGgmlQ8_0 ? 16 * hf : 0;
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
+    for (int i = 2 * k; i < 2 * k + 2; i++) {
         const int at = BB * i + off + ((i & 1) ? 2 : 0);  // a multiple of 4
-        const u32x4a v = *reinterpret_cast<const u32x4a *>(sb + at);
+        const u32x4a v = load_as<u32x4a>(sb + at);
         r.c[i] = make_uint4(v[0], v[1], v[2], v[3]);
-        if (!(i & 1)) r.t[i >> 1] = *reinterpret_cast<const uint32_t *>(sb + at + 16);
+        if (!(i & 1)) r.t[i >> 1] = load_as<uint32_t>(sb + at + 16);
         if constexpr (T == kGgmlQ5_0) {
             if (i & 1)
-                r.x[i >> 1] = *reinterpret_cast<const uint32_t *>(sb + at + 16);
+                r.x[i >> 1] = load_as<uint32_t>(sb + at + 16);
             else
-                r.y[i >> 1] = *reinterpret_cast<const uint32_t *>(sb + at + 20);
+                r.y[i >> 1] = load_as<uint32_t>(sb + at + 20);
         }
     }
+}
+template <int T>
+__device__ __forceinline__ void qb_load(QbRegs &r, const uint8_t *sb, int hf) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) qb_load_pair<T>(r, sb, hf, k);
 }
 
 // The lane's 16 code bytes of block i (4 words, byte 4w + b: code byte 4w + b of its share);
@@ -480,6 +519,189 @@ __device__ __forceinline__ void gemm_split_blocks(KqTiles (&sm)[2], const float 
         gemm_split_kq<T>(sm, xs, wb, nbat, tid, acc);
     else
         gemm_split_qb<T>(sm, xs, wb, nbat, tid, acc);
+}
+
+// ---- tiles of 64 rows (prefill) -------------------------------------------------------------
+
+// LDS of the tile loop: two chunks of 64 k of 64 x rows (hi/lo), rows unpadded, their eight
+// 16-byte slots permuted by row (kq_slot) so that the 16 rows of one phase of an operand read
+// cover all 64 banks; and for the K formats the f32 sums of every row's 8 sub-blocks, for two
+// super-blocks.
+struct KqRowTiles {
+    _Float16 hi[2][64][64];
+    _Float16 lo[2][64][64];
+    float xsum[2][64][8];
+};
+__device__ inline int kq_slot(int r, int s) { return 8 * (s ^ ((r >> 1) & 7)); }
+
+// The f32 sum of the 32 elements that four consecutive lanes hold (v: each lane's own 8).
+__device__ inline float kq_quad_sum(float v) {
+    v += dpp_f<0xB1>(v);  // quad_perm(1,0,3,2)
+    return v + dpp_f<0x4E>(v);  // quad_perm(2,3,0,1)
+}
+
+// 64 rows x 256 columns over nsb super-blocks of 256 k, 512 threads: wave w accumulates rows
+// 32 rb + .., columns 32 w + .. in acc[rb].  A block decoded once serves 64 rows here against 32
+// in the slice loops above, which spend twice as long on decoding (VALU) as on matrix
+// instructions: 2000 tokens, a block of 4096-wide projections, Q4_K 752 -> 551 us, Q5_K 849 -> 572,
+// Q8_0 1159 -> 589, Q4_0 939 -> 570, Q5_0 1401 -> 631.  LDS bounds it (every wave reads all x operands: 128 KB a
+// chunk at 128 bytes a clock, as long as the chunk's matrix work).  Eight waves of one weight row per lane rather than four of two: the latter
+// spill at two waves per SIMD, and a spilled register waits for every load in flight.
+// x goes through LDS in chunks of 64 k, one barrier a chunk; the block bytes of a lane's weight
+// row (wb, at super-block 0) are loaded straight into its registers L chunks ahead.  xs: the
+// staging thread's x row tid / 8 at element 8 (tid % 8) (a row past the tile's last one points at any
+// valid row).  Nothing in the loop is conditional (a skipped load would make every wait for
+// memory a wait for all of it): past the end the last super-block is loaded again.
+template <int T>
+__device__ __forceinline__ void gemm_tile_blocks(KqRowTiles &sm, const float *xs, const uint8_t *wb, int nsb,
+                                                 int tid, floatx16 (&acc)[2]) {
+    constexpr bool K = T == kGgmlQ4K || T == kGgmlQ5K;
+    constexpr int L = K ? 3 : 2;  // chunks of blocks in flight
+    const int lane = tid & 63, j = lane & 31, hf = lane >> 5;
+    const int si = tid >> 3, sc = tid & 7;
+    const DeqConstV dk;
+    zero(acc[0]);
+    zero(acc[1]);
+    const int last = nsb - 1;
+
+    float4 xa[2], xb[2];  // chunks of even and odd number
+    auto load_x = [&](float4 (&x)[2], int c) {
+        c = min(c, 4 * nsb - 1);
+#pragma unroll
+        for (int u = 0; u < 2; u++) x[u] = *reinterpret_cast<const float4 *>(xs + (size_t)c * kKC + 4 * u);
+    };
+    auto stage_x = [&](const float4 (&x)[2], int c) {
+        const int buf = c & 1;
+        half8 h, l;
+        split8(x[0], x[1], h, l);
+        *reinterpret_cast<half8 *>(&sm.hi[buf][si][kq_slot(si, sc)]) = h;
+        *reinterpret_cast<half8 *>(&sm.lo[buf][si][kq_slot(si, sc)]) = l;
+        if constexpr (K) {
+            const float v = kq_quad_sum(((x[0].x + x[0].y) + (x[0].z + x[0].w)) + ((x[1].x + x[1].y) + (x[1].z + x[1].w)));
+            if (!(sc & 3)) sm.xsum[(c >> 2) & 1][si][2 * (c & 3) + (sc >> 2)] = v;
+        }
+    };
+    // block bytes: K formats, chunk g's qs in kr.qs[g], the header (and qh) of the current
+    // super-block in kr and of the next in hdr / qh; the others, chunk g's block pair in qr
+    KqRegs kr;
+    QbRegs qr;
+    uint4 hdr, qh;
+    // the wave's first row as a scalar base (in the global address space: made from an integer,
+    // a plain pointer would be loaded from with flat instructions, whose waits are LDS waits too),
+    // the lanes' rows as 32-bit offsets from it
+    const uint64_t w0 = (uint64_t)wb;
+    const uint64_t first = ((uint64_t)__builtin_amdgcn_readfirstlane((int)(w0 >> 32)) << 32) |
+                           (uint32_t)__builtin_amdgcn_readfirstlane((int)w0);
+    const global_bytes base = reinterpret_cast<global_bytes>(first);
+    const uint32_t off = (uint32_t)(w0 - first);
+    auto load16 = [](global_bytes at) {
+        const u32x4 v = load_as<u32x4>(at);
+        return make_uint4(v[0], v[1], v[2], v[3]);
+    };
+    auto load_w = [&](int sb, int g) {
+        const global_bytes at = base + (size_t)min(sb, last) * KQ<T>::BYTES;
+        if constexpr (K)
+            kr.qs[g] = load16(at + (off + 16 * hf) + KQ<T>::QS + 32 * g);
+        else
+            qb_load_pair<T>(qr, at + off, hf, g);
+    };
+    auto load_hdr = [&](int sb) {
+        const global_bytes at = base + (size_t)min(sb, last) * KQ<T>::BYTES;
+        hdr = load16(at + off);
+        qh = T == kGgmlQ5K ? load16(at + (off + 16 * hf) + 16) : make_uint4(0u, 0u, 0u, 0u);
+    };
+    floatx16 t[2];
+    auto multiply = [&](int buf, int q, const half8 &b) {
+        const int s = 4 * (q >> 1) + 2 * hf + (q & 1);
+        half8 ah[2], al[2];
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++) {
+            const int r = 32 * rb + j;
+            ah[rb] = *reinterpret_cast<const half8 *>(&sm.hi[buf][r][kq_slot(r, s)]);
+            al[rb] = *reinterpret_cast<const half8 *>(&sm.lo[buf][r][kq_slot(r, s)]);
+        }
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++) t[rb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[rb], b, t[rb], 0, 0, 0);
+#pragma unroll
+        for (int rb = 0; rb < 2; rb++) t[rb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[rb], b, t[rb], 0, 0, 0);
+    };
+
+    load_x(xa, 0);
+    load_x(xb, 1);
+    if constexpr (K) load_hdr(0);
+#pragma unroll
+    for (int g = 0; g < L; g++) load_w(0, g);
+    stage_x(xa, 0);
+    load_x(xa, 2);
+    __syncthreads();
+    for (int sb = 0; sb < nsb; sb++) {
+        KqScales sk;
+        float dd, dm;
+        if constexpr (K) {
+            kr.hdr = hdr;
+            kr.qh = qh;
+            sk = kq_scales(hdr);
+            dd = (float)__builtin_bit_cast(_Float16, (uint16_t)(hdr.x & 0xFFFFu));
+            dm = -(float)__builtin_bit_cast(_Float16, (uint16_t)(hdr.x >> 16));
+        }
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const int buf = g & 1, c = 4 * sb + g;
+            // memory returns in order: x first, so that waiting for it (next chunk but one) waits
+            // for no block bytes that are needed later
+            stage_x(g & 1 ? xa : xb, c + 1);
+            load_x(g & 1 ? xa : xb, c + 3);
+            load_w(g + L < 4 ? sb : sb + 1, (g + L) & 3);
+            if (K && g == 0) load_hdr(sb + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (K) {
+                half8 b[4];
+                kq_operands<T>(kr, sk, g, b, dk);
+                if (g == 0) {
+                    zero(t[0]);
+                    zero(t[1]);
+                }
+#pragma unroll
+                for (int q = 0; q < 4; q++) multiply(buf, q, b[q]);
+                if (g == 3) {
+                    // the min product: the sums of row j's sub-blocks (split hi + lo) against m of
+                    // the column's; then d and dmin of the lane's column
+                    const half8 m = kq_min_operand(sk, hf);
+#pragma unroll
+                    for (int rb = 0; rb < 2; rb++) {
+                        const float *xr = sm.xsum[sb & 1][32 * rb + j];
+                        half8 sh, sl;
+                        split8(*reinterpret_cast<const float4 *>(xr), *reinterpret_cast<const float4 *>(xr + 4), sh, sl);
+                        floatx16 u;
+                        zero(u);
+                        u = __builtin_amdgcn_mfma_f32_32x32x16_f16(sh, m, u, 0, 0, 0);
+                        u = __builtin_amdgcn_mfma_f32_32x32x16_f16(sl, m, u, 0, 0, 0);
+#pragma unroll
+                        for (int e = 0; e < 16; e++)
+                            acc[rb][e] = __builtin_fmaf(dm, u[e], __builtin_fmaf(dd, t[rb][e], acc[rb][e]));
+                    }
+                }
+            } else {
+                float d[2];
+                qb_scales<T>(qr, g, hf, d[0], d[1]);
+#pragma unroll
+                for (int ii = 0; ii < 2; ii++) {
+                    half8 b[2];
+                    qb_operands<T>(qr, 2 * g + ii, hf, b, dk);
+                    zero(t[0]);
+                    zero(t[1]);
+#pragma unroll
+                    for (int u = 0; u < 2; u++) multiply(buf, 2 * ii + u, b[u]);
+#pragma unroll
+                    for (int rb = 0; rb < 2; rb++)
+#pragma unroll
+                        for (int e = 0; e < 16; e++) acc[rb][e] = __builtin_fmaf(d[ii], t[rb][e], acc[rb][e]);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);  // (the next staging's converts wait for its loads)
+            __syncthreads();
+        }
+    }
 }
 
 }  // namespace

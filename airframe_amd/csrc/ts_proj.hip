@@ -47,25 +47,35 @@ __device__ inline void proj_tile_of(const ProjArgs &p, int id, int &rt, int &ct,
 // 64-row tiles over all of K; the epilogue from the accumulators.  The residuals of a 32 x 32
 // block are loaded together before any of them is used (one by one, each a trip to memory, they
 // took as long as the whole product of a 96-long reduction: 51 us of 2048 x 6144 outputs).
-__global__ __launch_bounds__(256, 2) void proj_tile_kernel(ProjArgs p) {
-    __shared__ __align__(16) GemmTiles sm;
+// T: 0 for f16 rows (4 waves of 64 columns), else the GGUF block type (8 waves of 32).
+template <int T>
+__global__ __launch_bounds__(T == 0 ? 256 : 512, 2) void proj_tile_kernel(ProjArgs p) {
+    constexpr int CB = T == 0 ? 2 : 1;
+    __shared__ __align__(16) std::conditional_t<T == 0, GemmTiles, KqRowTiles> sm;
     int rt, ct, sp;
     proj_tile_of(p, blockIdx.x, rt, ct, sp);
     if (sp >= 1) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 31, hf = lane >> 5;
     const int row0 = 64 * rt, col0 = kPT * ct;
-    const int si = tid >> 2, sc = tid & 3;
-    const float *xs = p.a + (size_t)min(row0 + si, p.M - 1) * p.K + 8 * sc;
-    const _Float16 *ws[4];
+    floatx16 acc[2][CB];
+    if constexpr (T == 0) {
+        const int si = tid >> 2, sc = tid & 3;
+        const _Float16 *ws[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) ws[i] = p.w + (size_t)min(col0 + si + 64 * i, p.N - 1) * p.KW + 8 * sc;
-    floatx16 acc[2][2];
-    gemm_tile_core(sm, xs, ws, p.KW / kTK, p.K / kTK, tid, acc);
+        for (int i = 0; i < 4; i++) ws[i] = p.w + (size_t)min(col0 + si + 64 * i, p.N - 1) * p.KW + 8 * sc;
+        gemm_tile_core(sm, p.a + (size_t)min(row0 + si, p.M - 1) * p.K + 8 * sc, ws, p.KW / kTK, p.K / kTK, tid, acc);
+    } else {
+        floatx16 c[2];
+        gemm_tile_blocks<T>(sm, p.a + (size_t)min(row0 + (tid >> 3), p.M - 1) * p.K + 8 * (tid & 7),
+                            p.bw + (size_t)min(col0 + 32 * wave + j, p.N - 1) * p.brow, p.K / 256, tid, c);
+        acc[0][0] = c[0];
+        acc[1][0] = c[1];
+    }
 #pragma unroll
     for (int rb = 0; rb < 2; rb++)
 #pragma unroll
-        for (int cb = 0; cb < 2; cb++) {
-            const int col = col0 + 64 * wave + 32 * cb + j;
+        for (int cb = 0; cb < CB; cb++) {
+            const int col = col0 + 32 * (CB * wave + cb) + j;
             const int r0 = row0 + 32 * rb + 4 * hf;
             float res[16];
 #pragma unroll
@@ -206,11 +216,18 @@ ProjPlan proj_plan(int M, int K, int N) {
     return p;
 }
 
-ProjPlan proj_plan_kq(int M, int K, int N) {
+ProjPlan proj_plan_kq(int ggml_type, int M, int K, int N) {
     ProjPlan p;
     p.CT = (N + kPT - 1) / kPT;
     p.RT = (M + 31) / 32;
     const int tiles = p.RT * p.CT;
+    if (kq_tiles(ggml_type, tiles)) {
+        p.RT = (M + 63) / 64;
+        p.kps = K;
+        p.n_split = 1;
+        p.part_bytes = 0;
+        return p;
+    }
     // splits for about one workgroup per CU (256): measured on config 3's decode shapes, 512
     // and 1024 were no faster (the split count is capped at kMaxPSplit anyway)
     const int want = tiles < 256 ? std::min(kMaxPSplit, std::max(1, (256 + tiles - 1) / tiles)) : 1;
@@ -243,17 +260,14 @@ hipError_t launch_proj_kq(const float *a, int M, int K, int ggml_type, const voi
     p.n_split = plan.n_split;
     p.n_wg = plan.RT * plan.CT * plan.n_split;
     const int grid = (p.n_wg + 7) / 8 * 8;
-    if (ggml_type == kGgmlQ4K)
-        proj_split_kq_kernel<kGgmlQ4K><<<grid, 256, 0, st>>>(p);
-    else if (ggml_type == kGgmlQ5K)
-        proj_split_kq_kernel<kGgmlQ5K><<<grid, 256, 0, st>>>(p);
-    else if (ggml_type == kGgmlQ8_0)
-        proj_split_kq_kernel<kGgmlQ8_0><<<grid, 256, 0, st>>>(p);
-    else if (ggml_type == kGgmlQ5_0)
-        proj_split_kq_kernel<kGgmlQ5_0><<<grid, 256, 0, st>>>(p);
-    else
-        proj_split_kq_kernel<kGgmlQ4_0><<<grid, 256, 0, st>>>(p);
-    proj_reduce_kernel<<<plan.RT * plan.CT * (32 / kPRows), 256, 0, st>>>(p);
+    kq_dispatch(ggml_type, [&](auto tc) {
+        constexpr int T = decltype(tc)::value;
+        if (plan.part_bytes == 0)
+            proj_tile_kernel<T><<<grid, 512, 0, st>>>(p);
+        else
+            proj_split_kq_kernel<T><<<grid, 256, 0, st>>>(p);
+    });
+    if (plan.part_bytes > 0) proj_reduce_kernel<<<plan.RT * plan.CT * (32 / kPRows), 256, 0, st>>>(p);
     return hipGetLastError();
 }
 
@@ -279,7 +293,7 @@ hipError_t launch_proj(const float *a, int M, int K, const uint16_t *w, int N, f
     p.n_wg = plan.RT * plan.CT * plan.n_split;
     const int grid = (p.n_wg + 7) / 8 * 8;
     if (plan.n_split == 1) {
-        proj_tile_kernel<<<grid, 256, 0, st>>>(p);
+        proj_tile_kernel<0><<<grid, 256, 0, st>>>(p);
     } else {
         proj_split_kernel<<<grid, 256, 0, st>>>(p);
         proj_reduce_kernel<<<plan.RT * plan.CT * (32 / kPRows), 256, 0, st>>>(p);

@@ -320,11 +320,14 @@ __device__ inline void find_units(const QkvArgs &a, int u0, RowTile (&t)[N]) {
 // 64 x 64, 2 x 2 MFMA blocks: every weight operand feeds two row blocks and every x operand two
 // column blocks).  q goes out straight from the accumulators; for K and V the epilogue runs 32
 // rows at a time on a 32 x 256 LDS tile that reuses the operand buffers.
-__global__ __launch_bounds__(256, 2) void qkv_tile_kernel(QkvArgs a) {
-    constexpr int MT = 64, NU = MT / kMT;
+// T: 0 for f16 weight rows (4 waves of 64 columns, the epilogue one row block after the other),
+// else the GGUF block type (8 waves of 32 columns, four of them for the epilogue of either block).
+template <int T>
+__global__ __launch_bounds__(T == 0 ? 256 : 512, 2) void qkv_tile_kernel(QkvArgs a) {
+    constexpr int MT = 64, NU = MT / kMT, CB = T == 0 ? 2 : 1;
     union Smem {
-        GemmTiles x;
-        float tile[kMT][kTStr];
+        std::conditional_t<T == 0, GemmTiles, KqRowTiles> x;
+        float tile[T == 0 ? 1 : 2][kMT][kTStr];
     };
     __shared__ __align__(16) Smem sm;
     __shared__ RowTile t[NU];
@@ -347,17 +350,24 @@ __global__ __launch_bounds__(256, 2) void qkv_tile_kernel(QkvArgs a) {
     __syncthreads();
     if (!t[0].live) return;  // (units are live from the first one on)
 
-    // staging roles: x row si (an empty row reads the first unit's first live one)
-    const int si = tid >> 2, sc = tid & 3;
+    // staging role: x row si (an empty row reads the first unit's first live one)
+    const int si = tid / (T == 0 ? 4 : 8), sc = tid % (T == 0 ? 4 : 8);
     const RowTile us = t[si / kMT];
     int xr = us.live ? x_row(a, us, si % kMT) : -1;
     if (xr < 0) xr = x_row(a, t[0], a.n_tok == 1 ? 0 : t[0].lo - t[0].blk * kBlk);
     const float *xs = a.x + (size_t)xr * a.dim + 8 * sc;
-    const _Float16 *ws[4];
+    floatx16 acc[2][CB];
+    if constexpr (T == 0) {
+        const _Float16 *ws[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) ws[i] = w_row(a, ct, si + 64 * i) + 8 * sc;
-    floatx16 acc[2][2];
-    gemm_tile_core(sm.x, xs, ws, a.wld / kTK, a.dim / kTK, tid, acc);
+        for (int i = 0; i < 4; i++) ws[i] = w_row(a, ct, si + 64 * i) + 8 * sc;
+        gemm_tile_core(sm.x, xs, ws, a.wld / kTK, a.dim / kTK, tid, acc);
+    } else {
+        floatx16 c[2];
+        gemm_tile_blocks<T>(sm.x, xs, kq_row(a, ct, 32 * wave + j), a.dim / 256, tid, c);
+        acc[0][0] = c[0];
+        acc[1][0] = c[1];
+    }
 
     if (ct < a.n_qt) {
         const int ld = a.n_head * a.hd;
@@ -371,8 +381,8 @@ __global__ __launch_bounds__(256, 2) void qkv_tile_kernel(QkvArgs a) {
             const int hi = !u.live ? lo : single ? min(kMT, a.L.S - u.s) : u.hi - p0;
             const int64_t r0 = single ? u.s : (int64_t)u.s * a.n_tok + (p0 - u.start);
 #pragma unroll
-            for (int cb = 0; cb < 2; cb++) {
-                const int col = ct * kNT + 64 * wave + 32 * cb + j;
+            for (int cb = 0; cb < CB; cb++) {
+                const int col = ct * kNT + 32 * (CB * wave + cb) + j;
                 if (col >= ld) continue;
                 float *dst = a.q_out + (r0 + 4 * hf) * ld + col;
 #pragma unroll
@@ -384,23 +394,33 @@ __global__ __launch_bounds__(256, 2) void qkv_tile_kernel(QkvArgs a) {
         }
         return;
     }
-    // (the block index is a template constant, so that acc is indexed with constants and stays in
-    // registers)
-    auto block = [&](auto bc) {
-        constexpr int b = decltype(bc)::value;
-        const RowTile u = t[b];
-        if (!u.live) return;  // uniform
+    auto to_tile = [&](float (&tile)[kMT][kTStr], const floatx16 (&c)[CB]) {
 #pragma unroll
-        for (int cb = 0; cb < 2; cb++)
+        for (int cb = 0; cb < CB; cb++)
 #pragma unroll
-            for (int e = 0; e < 16; e++)
-                sm.tile[8 * (e >> 2) + 4 * hf + (e & 3)][64 * wave + 32 * cb + j] = acc[b][cb][e];
-        __syncthreads();
-        qkv_epilogue(a, u, ct, sm.tile, 0, kMT, tid);
-        __syncthreads();
+            for (int e = 0; e < 16; e++) tile[8 * (e >> 2) + 4 * hf + (e & 3)][32 * (CB * wave + cb) + j] = c[cb][e];
     };
-    block(std::integral_constant<int, 0>{});
-    block(std::integral_constant<int, 1>{});
+    if constexpr (T != 0) {
+        to_tile(sm.tile[0], acc[0]);
+        to_tile(sm.tile[1], acc[1]);
+        __syncthreads();
+        const RowTile u = t[tid >> 8];
+        if (u.live) qkv_epilogue(a, u, ct, sm.tile[tid >> 8], 0, kMT, tid & 255);  // (uniform for 4 waves)
+    } else {
+        // (the block index is a template constant, so that acc is indexed with constants and
+        // stays in registers)
+        auto block = [&](auto bc) {
+            constexpr int b = decltype(bc)::value;
+            const RowTile u = t[b];
+            if (!u.live) return;  // uniform
+            to_tile(sm.tile[0], acc[b]);
+            __syncthreads();
+            qkv_epilogue(a, u, ct, sm.tile[0], 0, kMT, tid);
+            __syncthreads();
+        };
+        block(std::integral_constant<int, 0>{});
+        block(std::integral_constant<int, 1>{});
+    }
 }
 
 // One split of the reduction for small grids (decode) through gemm_split_core; the f32
@@ -513,14 +533,22 @@ QkvPlan qkv_plan(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok) {
     return p;
 }
 
-QkvPlan qkv_plan_kq(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok) {
+QkvPlan qkv_plan_kq(int ggml_type, int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok) {
     QkvPlan p;
     const int hpt = 128 / hd;
     p.CT = (n_head * hd + kNT - 1) / kNT + (n_kv + hpt - 1) / hpt;
     p.big = false;
     p.RT = n_tok == 1 ? (n_seq + kMT - 1) / kMT : n_seq * (n_tok / kBlk + 2);
     const int tiles = p.RT * p.CT;
-    // few tiles: dim split over workgroups; many tiles: one slice over all of dim
+    if (kq_tiles(ggml_type, tiles)) {
+        p.big = true;
+        p.RT = (p.RT + 1) / 2;
+        p.kps = dim;
+        p.n_split = 1;
+        p.part_bytes = 0;
+        return p;
+    }
+    // few tiles: dim split over workgroups
     // splits for about one workgroup per CU (256): measured on config 3's decode shapes, 512
     // and 1024 were no faster (the split count is capped at kMaxSplit anyway)
     const int want = tiles < 256 ? std::min(kMaxSplit, std::max(1, (256 + tiles - 1) / tiles)) : 1;
@@ -565,16 +593,14 @@ hipError_t launch_qkv_kq(const KvLayerView &L, const int32_t *d_len, const float
     a.n_split = plan.n_split;
     a.n_wg = plan.RT * plan.CT * plan.n_split;
     const int grid = (a.n_wg + 7) / 8 * 8;
-    if (ggml_type == kGgmlQ4K)
-        qkv_split_kq_kernel<kGgmlQ4K><<<grid, 256, 0, st>>>(a);
-    else if (ggml_type == kGgmlQ5K)
-        qkv_split_kq_kernel<kGgmlQ5K><<<grid, 256, 0, st>>>(a);
-    else if (ggml_type == kGgmlQ8_0)
-        qkv_split_kq_kernel<kGgmlQ8_0><<<grid, 256, 0, st>>>(a);
-    else if (ggml_type == kGgmlQ5_0)
-        qkv_split_kq_kernel<kGgmlQ5_0><<<grid, 256, 0, st>>>(a);
-    else
-        qkv_split_kq_kernel<kGgmlQ4_0><<<grid, 256, 0, st>>>(a);
+    kq_dispatch(ggml_type, [&](auto tc) {
+        constexpr int T = decltype(tc)::value;
+        if (plan.big)
+            qkv_tile_kernel<T><<<grid, 512, 0, st>>>(a);
+        else
+            qkv_split_kq_kernel<T><<<grid, 256, 0, st>>>(a);
+    });
+    if (plan.big) return hipGetLastError();
     if (n_tok == 1)
         qkv_reduce_kernel<4><<<plan.RT * plan.CT * (kMT / 4), 256, 0, st>>>(a);
     else
@@ -616,7 +642,7 @@ hipError_t launch_qkv(const KvLayerView &L, const int32_t *d_len, const float *x
     a.n_wg = plan.RT * plan.CT * plan.n_split;
     const int grid = (a.n_wg + 7) / 8 * 8;
     if (plan.big) {
-        qkv_tile_kernel<<<grid, 256, 0, st>>>(a);
+        qkv_tile_kernel<0><<<grid, 256, 0, st>>>(a);
     } else {
         qkv_split_kernel<<<grid, 256, 0, st>>>(a);
         if (n_tok == 1)

@@ -2,16 +2,19 @@
 wrong: reductions of one to a few 32-long chunks and every remainder of the loop's three
 buffers, row counts around the 64-row tile, column counts around the 256-column tile, V blocks
 of several ragged sequences inside one row tile (also more than 64 sequences, which the unit
-search takes 64 at a time), and two weight planes.  Against the oracle's f32 dot within
+search takes 64 at a time), two weight planes, and GGUF blocks with so many tiles that the tile
+kernel takes them (one to three super-blocks).  Against the oracle's f32 dot within
 |err| <= 2e-3 + 1e-3*|ref|; cache codes bit-exact with the append of the kernel's own K and V."""
 import numpy as np
 import pytest
 import torch
 
-from airframe_amd.kv_cache import attn_out_proj
+from airframe_amd import weights
+from airframe_amd.kv_cache import attn_out_proj, attn_out_proj_gguf
 from oracle import oracle
 from tests.gpu_util import Pair, assert_close, dev, say
 from tests.test_gpu_qkv import run_case
+from tests.test_gpu_weights import random_blob
 
 pytestmark = pytest.mark.gpu
 
@@ -50,5 +53,52 @@ def test_out_proj_tiles(gpu, n_tok, attn_dim, dim, planes):
     attn_out_proj(dev(a), dev(wo), act_d, stash=stash_d, planes=planes)
     torch.cuda.synchronize()
     dot = oracle.project_f32(a, wf)
+    assert_close(stash_d.cpu().numpy(), dot, "projection")
+    assert_close(act_d.cpu().numpy(), act + dot, "residual + projection")
+
+
+@pytest.mark.parametrize("fmt,n_seq,n_tok,dim,n_head,n_kv,hd", [
+    (weights.Q4_K, 70, 3, 256, 2, 1, 64),
+    (weights.Q5_K, 65, 3, 768, 2, 1, 64),
+    (weights.Q8_0, 70, 35, 512, 2, 1, 64),
+    (weights.Q4_0, 33, 100, 256, 4, 2, 128),
+    (weights.Q5_0, 70, 5, 512, 3, 1, 128),
+])
+def test_qkv_block_tiles(gpu, fmt, n_seq, n_tok, dim, n_head, n_kv, hd):
+    say(f"qkv block tiles fmt={fmt} n_seq={n_seq} n_tok={n_tok} dim={dim} n_head={n_head} n_kv={n_kv} hd={hd}")
+    rng = np.random.default_rng(fmt + dim + n_tok)
+    p = Pair(n_seq, n_kv, hd, 100 + n_tok, 1e6)
+    p.set_lens(rng.integers(0, 97, size=n_seq).astype(np.int32))
+    rows = (n_head * hd, n_kv * hd, n_kv * hd)
+    blobs = [random_blob(rng, fmt, r, dim) for r in rows]
+    x = rng.standard_normal((n_seq, n_tok, dim)).astype(np.float32)
+    k_out = torch.empty((n_seq, n_tok, n_kv, hd), dtype=torch.float32, device="cuda")
+    v_out = torch.empty_like(k_out)
+    q = p.gpu.qkv_append_gguf(0, dev(x), fmt, *(dev(b) for b in blobs), p.rope, kv_out=(k_out, v_out))
+    torch.cuda.synchronize()
+    q, k_out, v_out = q.cpu().numpy(), k_out.cpu().numpy(), v_out.cpu().numpy()
+    xf = x.reshape(-1, dim)
+    for name, got, blob, r in (("q", q, blobs[0], rows[0]), ("k", k_out, blobs[1], rows[1]), ("v", v_out, blobs[2], rows[2])):
+        ref = oracle.project_f32(xf, oracle.dequant(fmt, blob, r * dim).reshape(r, dim))
+        assert_close(got.reshape(n_seq * n_tok, -1), ref, name)
+    p.ora.append(k_out, v_out)
+    p.advance(n_tok)
+    p.check_codes()
+
+
+@pytest.mark.parametrize("fmt,n_tok,attn_dim,dim", [
+    (weights.Q4_K, 900, 256, 2049), (weights.Q5_K, 8195, 256, 8), (weights.Q8_0, 830, 512, 1800),
+    (weights.Q4_0, 900, 768, 2300), (weights.Q5_0, 641, 256, 2560),
+])
+def test_out_proj_block_tiles(gpu, fmt, n_tok, attn_dim, dim):
+    say(f"out_proj block tiles fmt={fmt} n_tok={n_tok} attn_dim={attn_dim} dim={dim}")
+    rng = np.random.default_rng(fmt + n_tok + dim)
+    blob = random_blob(rng, fmt, dim, attn_dim)
+    a = rng.standard_normal((n_tok, attn_dim)).astype(np.float32)
+    act = (rng.standard_normal((n_tok, dim)) * 4).astype(np.float32)
+    act_d, stash_d = dev(act), torch.zeros((n_tok, dim), dtype=torch.float32, device="cuda")
+    attn_out_proj_gguf(dev(a), fmt, dev(blob), dim, act_d, stash=stash_d)
+    torch.cuda.synchronize()
+    dot = oracle.project_f32(a, oracle.dequant(fmt, blob, dim * attn_dim).reshape(dim, attn_dim))
     assert_close(stash_d.cpu().numpy(), dot, "projection")
     assert_close(act_d.cpu().numpy(), act + dot, "residual + projection")
