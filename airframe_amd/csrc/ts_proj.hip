@@ -8,12 +8,14 @@
 // act = act + dot (:818-820).  Same matrix-core loops as the QKV projection (ts_gemm.h):
 //   * enough 64-row tiles: one workgroup per 64 x 256 tile over all of attn_dim, the result
 //     added to act straight from the accumulators;
+//   * one or two rows: ts_gemv.h, one kernel;
 //   * few tiles (decode): 32 x 256 tiles with attn_dim split across workgroups (f32
 //     partials), then a kernel that sums the partials in split order and adds them to act.
 // Taking the combine's output rather than the decode partials is deliberate: every column
 // tile reads all of a token's attention output, so folding the combine into this kernel would
 // redo it (n_split-fold reads of the partials) once per column tile.
 #include "ts_gemm.h"
+#include "ts_gemv.h"
 #include "ts_internal.h"
 #include "ts_kquant.h"
 
@@ -143,6 +145,38 @@ __global__ __launch_bounds__(256) void proj_split_kq_kernel(ProjArgs p) {
             dst[(8 * (e >> 2) + 4 * hf + (e & 3)) * kPT + 64 * wave + 32 * cb + j] = acc[cb][e];
 }
 
+// One or two rows (decode): 8 R output columns per workgroup, complete in one kernel (ts_gemv.h).
+template <int T, int MB, int R>
+__global__ __launch_bounds__(256) void proj_gemv_kernel(ProjArgs p) {
+    extern __shared__ __align__(16) float sx[];
+    __shared__ float red[4 * 8 * R * MB];
+    const int tid = threadIdx.x, g = (tid & 63) >> 3;
+    const int n0 = (blockIdx.x * 8 + g) * R;
+    const uint8_t *row[R];
+    float res[R][MB], out[R][MB];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int n = min(n0 + r, p.N - 1);
+        if constexpr (T == kGemvF16 || T == kGemvF16x2)
+            row[r] = reinterpret_cast<const uint8_t *>(p.w + (size_t)n * p.KW);
+        else
+            row[r] = p.bw + (size_t)n * p.brow;
+#pragma unroll
+        for (int m = 0; m < MB; m++) res[r][m] = tid < 64 ? p.act[(size_t)min(m, p.M - 1) * p.N + n] : 0.0f;
+    }
+    gemv_rows<T, MB, R>(sx, red, p.a, p.M, p.K, p.K, row, (size_t)p.K * 2, tid, out);
+    if (tid >= 64 || (tid & 7)) return;
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int m = 0; m < MB; m++) {
+            if (n0 + r >= p.N || m >= p.M) continue;
+            const size_t i = (size_t)m * p.N + n0 + r;
+            if (p.stash) p.stash[i] = out[r][m];
+            p.act[i] = res[r][m] + out[r][m];
+        }
+}
+
 // Sum of the partials of NR rows of one tile in split order, added to act.
 constexpr int kPRows = 4;  // rows per workgroup of the sum (4 vs 8: config 3 14.1 vs 15.0 us, config 2 11.5 vs 12.2)
 __global__ __launch_bounds__(256) void proj_reduce_kernel(ProjArgs p) {
@@ -183,6 +217,13 @@ __global__ __launch_bounds__(256) void fill_zero_kernel(float4 *p, size_t n4) {
 }
 
 }  // namespace
+
+static void proj_gemv(int t, const ProjArgs &p, hipStream_t st) {
+    gemv_dispatch(t, gemv_mb(p.M), [&](auto tc, auto mc) {
+        constexpr int T = decltype(tc)::value, MB = decltype(mc)::value, R = gemv_r(MB);
+        proj_gemv_kernel<T, MB, R><<<(p.N + 8 * R - 1) / (8 * R), 256, gemv_lds(MB, p.K), st>>>(p);
+    });
+}
 
 // Zeroes n floats (n a multiple of 4, p 16-byte aligned) with a kernel, so that a caller may
 // capture it in a graph.
@@ -259,6 +300,10 @@ hipError_t launch_proj_kq(const float *a, int M, int K, int ggml_type, const voi
     p.kps = plan.kps;
     p.n_split = plan.n_split;
     p.n_wg = plan.RT * plan.CT * plan.n_split;
+    if (gemv_fits(M, K) && plan.part_bytes > 0) {
+        proj_gemv(ggml_type, p, st);
+        return hipGetLastError();
+    }
     const int grid = (p.n_wg + 7) / 8 * 8;
     kq_dispatch(ggml_type, [&](auto tc) {
         constexpr int T = decltype(tc)::value;
@@ -294,6 +339,8 @@ hipError_t launch_proj(const float *a, int M, int K, const uint16_t *w, int N, f
     const int grid = (p.n_wg + 7) / 8 * 8;
     if (plan.n_split == 1) {
         proj_tile_kernel<0><<<grid, 256, 0, st>>>(p);
+    } else if (gemv_fits(M, K)) {
+        proj_gemv(planes == 2 ? kGemvF16x2 : kGemvF16, p, st);
     } else {
         proj_split_kernel<<<grid, 256, 0, st>>>(p);
         proj_reduce_kernel<<<plan.RT * plan.CT * (32 / kPRows), 256, 0, st>>>(p);

@@ -22,10 +22,12 @@
 // block of one sequence (the block owns its V words, as in the append kernel).
 //   * Enough tiles (prefill, large batches): one workgroup per 64-row tile over all of dim
 //     (gemm_tile_core), the epilogue on the finished tile.
+//   * One or two sequences, one token each: ts_gemv.h, then the append kernel.
 //   * Few tiles (decode): 32-row tiles with the reduction over dim split across workgroups
 //     (gemm_split_core, one memory round trip per slice), f32 partials, and a second kernel
 //     that sums them in split order (deterministic) and runs the epilogue.
 #include "ts_gemm.h"
+#include "ts_gemv.h"
 #include "ts_kquant.h"
 #include "ts_store.h"
 
@@ -502,6 +504,57 @@ __global__ __launch_bounds__(256) void qkv_reduce_kernel(QkvArgs a) {
     qkv_epilogue(a, t, ct, tile, r0, NR, tid);
 }
 
+// One or two sequences, one new token each (ts_gemv.h): 8 R of the q, K and V rows per workgroup; q to the
+// caller, K and V as f32 to k_out and v_out, which the append kernel quantizes next.
+template <int T, int MB, int R>
+__global__ __launch_bounds__(256) void qkv_gemv_kernel(QkvArgs a) {
+    extern __shared__ __align__(16) float sx[];
+    __shared__ float red[4 * 8 * R * MB];
+    const int tid = threadIdx.x, g = (tid & 63) >> 3;
+    const int nq = a.n_head * a.hd, nk = a.L.H * a.hd, N = nq + 2 * nk;
+    const int n0 = (blockIdx.x * 8 + g) * R;  // (nq, nk multiples of 64: R rows never straddle)
+    const uint8_t *row[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int n = min(n0 + r, N - 1);
+        const int w = n < nq ? 0 : n < nq + nk ? 1 : 2;
+        const size_t i = n - (w == 0 ? 0 : w == 1 ? nq : nq + nk);
+        if constexpr (T == kGemvF16 || T == kGemvF16x2)
+            row[r] = reinterpret_cast<const uint8_t *>((w == 0 ? a.wq : w == 1 ? a.wk : a.wv) + i * a.wld);
+        else
+            row[r] = (w == 0 ? a.bq : w == 1 ? a.bk : a.bv) + i * a.brow;
+    }
+    float out[R][MB];
+    gemv_rows<T, MB, R>(sx, red, a.x, a.L.S, a.dim, a.dim, row, (size_t)a.dim * 2, tid, out);
+    if (tid >= 64 || (tid & 7) || n0 >= N) return;
+    const int w = n0 < nq ? 0 : n0 < nq + nk ? 1 : 2;
+    float *dst = w == 0 ? a.q_out : w == 1 ? a.k_out : a.v_out;
+    const int ld = w == 0 ? nq : nk, c = n0 - (w == 0 ? 0 : w == 1 ? nq : nq + nk);
+#pragma unroll
+    for (int m = 0; m < MB; m++)
+        if (m < a.L.S) {
+#pragma unroll
+            for (int r = 0; r < R; r++) dst[(size_t)m * ld + c + r] = out[r][m];
+        }
+}
+
+// The projections of a few rows into q_out and f32 K and V (the caller's, or in part), then
+// their append.
+hipError_t qkv_gemv(int t, QkvArgs a, float *part, hipStream_t st) {
+    if (!a.k_out) {
+        a.k_out = part;
+        a.v_out = part + (size_t)a.L.S * a.L.H * a.hd;
+    }
+    const int N = (a.n_head + 2 * a.L.H) * a.hd;
+    gemv_dispatch(t, gemv_mb(a.L.S), [&](auto tc, auto mc) {
+        constexpr int T = decltype(tc)::value, MB = decltype(mc)::value, R = gemv_r(MB);
+        qkv_gemv_kernel<T, MB, R><<<(N + 8 * R - 1) / (8 * R), 256, gemv_lds(MB, a.dim), st>>>(a);
+    });
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    return launch_quantize_rows(a.L, a.k_out, a.v_out, a.len, 0, 1, 1, a.rope, a.rope_pairs, 1, st);
+}
+
 }  // namespace
 
 QkvPlan qkv_plan(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok) {
@@ -592,6 +645,7 @@ hipError_t launch_qkv_kq(const KvLayerView &L, const int32_t *d_len, const float
     a.kps = plan.kps;
     a.n_split = plan.n_split;
     a.n_wg = plan.RT * plan.CT * plan.n_split;
+    if (n_tok == 1 && gemv_fits(L.S, dim) && !plan.big) return qkv_gemv(ggml_type, a, part, st);
     const int grid = (a.n_wg + 7) / 8 * 8;
     kq_dispatch(ggml_type, [&](auto tc) {
         constexpr int T = decltype(tc)::value;
@@ -640,6 +694,9 @@ hipError_t launch_qkv(const KvLayerView &L, const int32_t *d_len, const float *x
     a.kps = plan.kps;
     a.n_split = plan.n_split;
     a.n_wg = plan.RT * plan.CT * plan.n_split;
+    // (the split plans' scratch is at least 256 floats for every K and V column of 32 rows)
+    if (n_tok == 1 && gemv_fits(L.S, dim) && !plan.big)
+        return qkv_gemv(planes == 2 ? kGemvF16x2 : kGemvF16, a, part, st);
     const int grid = (a.n_wg + 7) / 8 * 8;
     if (plan.big) {
         qkv_tile_kernel<0><<<grid, 256, 0, st>>>(a);
