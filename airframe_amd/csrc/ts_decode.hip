@@ -1394,18 +1394,13 @@ windows_done:
 
 }  // namespace
 
-// Split plan.  The integer kernel (G <= 8) runs one workgroup per CU (4 waves, 8 for 64-dim
-// rows), the 16x16 kernel two per CU.  The chunk (positions per split, a multiple of 64) is the smallest one for which
-// the busy workgroups of the whole batch, n_kv * sum_s ceil(n_ctx[s] / chunk), fit in that
-// target: the batch's total context spread evenly, so ragged batches give their long
-// sequences more splits and no CU gets a second workgroup.  (Measured on the config-3 shape
-// with a loads-only probe of the same access pattern: one workgroup per stream and CU 43.2 us,
-// two 44.7 us, three 45.6 us.)  Splits shorter than kMinChunk leave waves without a window.
 namespace {
-constexpr int kMinChunk = 256;
-constexpr int kG4MinChunk = 1024;  // the integer kernel needs >= 4 windows per wave to pay off
+constexpr int kMinChunk = 256;  // splits shorter than this leave waves without a window
 
-int plan_chunk(const int32_t *n_ctx, int n_seq, int n_kv, int target) {
+// The chunk that spreads a batch's context evenly: the smallest multiple of 64 for which the busy
+// workgroups of the whole batch, n_kv * sum_s ceil(n_ctx[s] / chunk), fit in `target`; with
+// more streams than the target, the batch's work over the target.
+int even_chunk(const int32_t *n_ctx, int n_seq, int n_kv, int target) {
     int64_t total = 0;
     int max_ctx = 1;
     for (int s = 0; s < n_seq; s++) {
@@ -1420,60 +1415,149 @@ int plan_chunk(const int32_t *n_ctx, int n_seq, int n_kv, int target) {
     const int hi_c = std::max(kMinChunk, (max_ctx + 63) / 64 * 64);
     int lo_c = (int)std::min<int64_t>(hi_c, std::max<int64_t>(kMinChunk, (total * n_kv + target - 1) / target));
     lo_c = (lo_c + 63) / 64 * 64;
-    // smallest multiple of 64 in [lo_c, hi_c] with busy <= target (busy is non-increasing)
-    int lo = lo_c / 64, hi = hi_c / 64;
+    int lo = lo_c / 64, hi = hi_c / 64;  // busy is non-increasing
     while (lo < hi) {
         const int mid = (lo + hi) / 2;
         if (busy(64 * mid) <= target) hi = mid; else lo = mid + 1;
     }
-    // More streams than the target (many sequences): no chunk meets it.  The balanced chunk
-    // (the batch's work over the target) still splits the sequences much longer than the rest,
-    // which would otherwise stream alone after the others finished; for a uniform batch it is
-    // the whole sequence anyway.
     if (busy(64 * lo) > target) return lo_c;
     return 64 * lo;
 }
+
+// What the plan weighs, in us, of either kernel: a workgroup's fixed part (lengths, q operands,
+// the merge of its waves), one round of its waves (a 64-position window each, `span` positions
+// together) and how many workgroups run at once.  From times of splits of 64 positions to whole
+// sequences of 1 to 32 sequences of 60 to 32K positions (time against rounds of the longest
+// split), all head shapes.
+struct DecodeCost {
+    float fixed, round;
+    int span;
+    float at_once;
+};
+// The integer kernel: one workgroup per CU; a second half of query heads makes a round half as long
+// again, four halves 2.5 times (their QK^T and softmax share the wave), and all lengthen the
+// fixed part (their q digits and merges).
+DecodeCost int_cost(int G, int hd, int n_cu) {
+    const int halves = (G + 3) / 4;
+    const float heads = halves <= 1 ? 1.0f : halves == 2 ? 1.5f : 2.5f;
+    const float fixed = halves <= 1 ? 5.0f : halves == 2 ? 7.5f : 13.0f;
+    if (hd == 64) return {fixed, (halves <= 1 ? 1.4f : halves == 2 ? 1.8f : 3.2f), 512, (float)n_cu};
+    if (hd == 256) return {fixed + 2.5f, 1.75f * heads, 256, (float)n_cu};
+    return {fixed, 0.95f * heads, 256, (float)n_cu};
+}
+// The 16x16 kernel: two workgroups fit a CU but get in each other's way (together 1.25 times one).
+DecodeCost f16_cost(int G, int hd, int n_cu) {
+    const float heads = G > 4 ? 1.4f : 1.0f;
+    return {4.0f, (hd == 64 ? 1.33f : hd == 128 ? 1.55f : 3.2f) * heads, 256, 1.25f * n_cu};
+}
+constexpr float kCombineUs = 3.5f;        // the combine launch behind a plan with splits
+constexpr float kDecodeBytesUs = 6.5e6f;  // bytes a us that all CUs stream together
+
+// Estimated time of a plan with splits of `chunk`: the longest split, or the batch's work over the
+// workgroups that run at once (the last to start then ends half a split later on average), or
+// the bytes.  Only 7/8 of the CUs count when the grid holds idle workgroups (splits past a
+// shorter sequence's end): busy ones then wait 9-20 us for a CU that others leave, since the
+// dispatcher does not place a workgroup on just any free CU of its XCD.
+float plan_us(const DecodeCost &k, const int32_t *n_ctx, int n_seq, int streams, int64_t total, int max_ctx, int chunk,
+              int n_cu, float bytes_us) {
+    const float inv = 1.0f / chunk;
+    const int most = (max_ctx + chunk - 1) / chunk;
+    int64_t n = 0;
+    bool idle = false;
+    for (int s = 0; s < n_seq; s++) {
+        const int c = (int)((n_ctx[s] - 0.5f) * inv) + 1;
+        n += c;
+        idle |= c != most;
+    }
+    const float cus = idle ? 0.875f : 1.0f;
+    const float longest = k.fixed + k.round * ((std::min(chunk, max_ctx) + k.span - 1) / k.span);
+    float us = longest;
+    if (n * streams > cus * n_cu) {
+        const float work = n * streams * (k.fixed + 0.5f * k.round) + k.round * total * streams / k.span;
+        us = std::max(us, work / (cus * k.at_once) + 0.5f * longest);
+    }
+    return std::max(us, bytes_us + k.fixed) + (most > 1 ? kCombineUs : 0.0f);
+}
 }  // namespace
 
-DecodePlan decode_plan(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_cu, int stored_hd, bool fused) {
-    const int int_gmax = decode_int_gmax(stored_hd);
+// The batch's context spread evenly (even_chunk) over 7/8 of the CUs for the integer kernel, or, when
+// its splits would be short, over twice the CUs for the 16x16 kernel.
+DecodePlan decode_plan_even(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_cu, int stored_hd) {
     DecodePlan p;
     p.nw = 4;
+    p.g4 = false;
     int max_ctx = 1;
     for (int s = 0; s < n_seq; s++) max_ctx = std::max(max_ctx, (int)n_ctx[s]);
-    p.g4 = false;
-    if (G <= int_gmax) {  // the integer kernel: one, two or four halves of 4 query heads
-        // Target 7/8 of the CUs, not all of them: a plan that fills every CU of a ragged
-        // batch had ~24 busy workgroups wait 9-20 us for a CU (behind busy ones) while idle
-        // splits freed others -- the dispatcher does not place a workgroup on just any free
-        // CU of its XCD.  Over ten length draws of config 4: 0.441-0.679 of HBM peak (mean
-        // 0.60) with every CU, 0.648-0.682 (mean 0.66) with 7/8.  Uniform batches (one split
-        // per stream, config 3) are not affected.
-        p.chunk = plan_chunk(n_ctx, n_seq, n_kv, n_cu - n_cu / 8);
-        p.g4 = p.chunk >= kG4MinChunk;
+    if (G <= decode_int_gmax(stored_hd)) {
+        p.chunk = even_chunk(n_ctx, n_seq, n_kv, n_cu - n_cu / 8);
+        p.g4 = p.chunk >= 1024;
     }
-    // the 16x16 kernel takes up to 8 query heads per workgroup: more as several head groups
-    if (!p.g4) p.chunk = plan_chunk(n_ctx, n_seq, n_kv * ((G + 7) / 8), 2 * n_cu);
+    if (!p.g4) p.chunk = even_chunk(n_ctx, n_seq, n_kv * ((G + 7) / 8), 2 * n_cu);
     p.n_split = (max_ctx + p.chunk - 1) / p.chunk;
-    // Few streams, short context: one wide workgroup per stream instead of a split, when its
-    // waves cover the longest sequence's windows (the positions before the new token with the
-    // fused append, which scores that one from registers) in one round.  No combine launch
-    // (the split kernel then also advances the lengths), the merge stays in LDS.  The fewest
-    // waves that cover it: 8 waves measured 9.1 us per step on config 1's shape (512 positions
-    // + the new token), 16 waves 10.1, four-wave splits and a combine 10.5.  More than one
-    // window per wave does not pay: 8.5 windows per wave took 26.6 us per layer on config 2's
+    return p;
+}
+
+// Split plan: the kernel and the split length whose estimate is the lowest, among the batch's
+// context spread evenly (decode_plan_even) and equal shares of the longest sequence, fewest first;
+// a later one in that order has to gain 2%.  (The even plan alone gave a ragged batch of about as
+// many streams as CUs a few second splits, which waited for the first ones, with a combine behind
+// them and idle workgroups between.  32 sequences of 700-1531 positions, 8 kv heads: 27.3 us with
+// two splits for some, 17.8 with none; 2000-6000: 36.4, 30.1; 64-dim rows, 1000-3000: 22.1, 13.2.
+// And the integer kernel took only splits of 1024 and more: 8 sequences of 1000-4000 positions
+// with 256-dim rows 36.2 us on the 16x16 kernel, 19.3 in integer splits of 832; one sequence of
+// 20000 with 24 query heads 17.2 us a layer, 12.4.)
+DecodePlan decode_plan(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_cu, int stored_hd, bool fused) {
+    int max_ctx = 1;
+    int64_t total = 0;
+    for (int s = 0; s < n_seq; s++) {
+        max_ctx = std::max(max_ctx, (int)n_ctx[s]);
+        total += n_ctx[s];
+    }
+    DecodePlan p;
+    p.nw = 4;
+    const int groups = (G + 7) / 8;  // head groups of the 16x16 kernel
+    // Few streams, short context: one wide workgroup of the 16x16 kernel per stream instead of a
+    // split, when its waves cover the longest sequence's windows (the positions before the new
+    // token with the fused append, which scores that one from registers) in one round.  No
+    // combine launch (the split kernel then also advances the lengths), the merge stays in LDS.
+    // The fewest waves that cover it: 8 waves measured 9.1 us per step on config 1's shape (512
+    // positions + the new token), 16 waves 10.1, four-wave splits and a combine 10.5.  More than
+    // one window per wave does not pay: 8.5 windows per wave took 26.6 us per layer on config 2's
     // shape against 10.0 with splits and a combine.
     const int n_win = (max_ctx - (fused ? 1 : 0) + 63) / 64;
-    if (!p.g4 && n_win > 4 && (int64_t)n_seq * n_kv * ((G + 7) / 8) <= n_cu) {
-        const int wmax = stored_hd <= 64 ? 16 : stored_hd <= 128 ? 8 : 4;
-        for (int nw = 8; nw <= wmax; nw *= 2)
-            if (n_win <= nw) {
-                p.nw = nw;
-                p.chunk = (max_ctx + 63) / 64 * 64;
-                p.n_split = 1;
-                break;
-            }
+    const int wmax = stored_hd <= 64 ? 16 : stored_hd <= 128 ? 8 : 4;
+    if (n_win > 4 && n_win <= wmax && (int64_t)n_seq * n_kv * groups <= n_cu) {
+        p.g4 = false;
+        p.nw = n_win <= 8 ? 8 : 16;
+        p.chunk = (max_ctx + 63) / 64 * 64;
+        p.n_split = 1;
+        return p;
     }
+    const float bytes_us = (float)total * n_kv * (stored_hd + 8) / kDecodeBytesUs;
+    const bool integer = G <= decode_int_gmax(stored_hd);
+    const DecodeCost ki = int_cost(G, stored_hd, n_cu), kf = f16_cost(G, stored_hd, n_cu);
+    float best = 0.0f;
+    p.chunk = 0;
+    auto weigh = [&](int chunk, bool g4) {
+        const float us = g4 ? plan_us(ki, n_ctx, n_seq, n_kv, total, max_ctx, chunk, n_cu, bytes_us)
+                            : plan_us(kf, n_ctx, n_seq, n_kv * groups, total, max_ctx, chunk, n_cu, bytes_us);
+        if (p.chunk == 0 || us < 0.98f * best) {
+            best = us;
+            p.g4 = g4;
+            p.chunk = chunk;
+        }
+    };
+    const DecodePlan even = decode_plan_even(n_ctx, n_seq, n_kv, G, n_cu, stored_hd);
+    weigh(even.chunk, even.g4);
+    const int most = std::min((max_ctx + kMinChunk - 1) / kMinChunk, decode_cap(n_kv, max_ctx, n_cu));
+    for (int k = 1; k <= most; k = k == most ? k + 1 : std::min(most, k + (k < 8 ? 1 : k / 4))) {
+        // (a few positions to spare, so that the plan of a length that is a multiple of k windows
+        // outlives the next tokens, as a captured one has to)
+        const int chunk = ((max_ctx + k - 1) / k + (k > 1 ? 4 : 0) + 63) / 64 * 64;
+        if (integer) weigh(chunk, true);
+        weigh(chunk, false);
+    }
+    p.n_split = (max_ctx + p.chunk - 1) / p.chunk;
     return p;
 }
 

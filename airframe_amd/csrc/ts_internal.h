@@ -160,6 +160,9 @@ struct DecodePlan {
 // stored_hd: the stored head dim (64, 128 or 256); fused: the launch appends the new token
 // (its position is scored from registers, not streamed).
 DecodePlan decode_plan(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_cu, int stored_hd, bool fused);
+// The plan that ts_attn_decode_append_noalloc falls back to when the partials of decode_plan's do
+// not fit its scratch array: fewer splits for some batches.
+DecodePlan decode_plan_even(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_cu, int stored_hd);
 // The integer kernel takes up to 16 query heads per kv head on stored rows up to 128 dims, 8 on
 // 256-dim rows.
 inline int decode_int_gmax(int stored_hd) { return stored_hd <= 128 ? 16 : 8; }

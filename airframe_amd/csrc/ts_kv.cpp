@@ -473,10 +473,14 @@ static int attn_decode(const ts_kv *kv, int32_t layer, const float *d_q, int32_t
     for (int s = 0; s < kv->d.n_seq; s++) ctx[s] = kv->h_len[s] + 1;
     ts::DecodePlan plan = ts::decode_plan(ctx.data(), kv->d.n_seq, kv->d.n_head_kv, n_head / kv->d.n_head_kv,
                                           kv->n_cu, kv->hdp, k_new != nullptr);
+    // partials [S][n_head][n_split][hd], then m and l [S][n_head][n_split]
+    const uint64_t per_split = (uint64_t)kv->d.n_seq * n_head * (kv->hdp + 2) * sizeof(float);
+    if (noalloc && plan.n_split > 1 && plan.n_split * per_split > workspace_bytes)
+        plan = ts::decode_plan_even(ctx.data(), kv->d.n_seq, kv->d.n_head_kv, n_head / kv->d.n_head_kv, kv->n_cu, kv->hdp);
     if (plan.n_split > 1) {
         uint64_t need = 0;
-        if (noalloc)  // partials [S][n_head][n_split][hd], then m and l [S][n_head][n_split]
-            need = (uint64_t)kv->d.n_seq * n_head * plan.n_split * (kv->hdp + 2) * sizeof(float);
+        if (noalloc)
+            need = plan.n_split * per_split;
         else  // plan.n_split <= decode_cap(max_seq), the count the workspace was sized for
             ts_attn_decode_workspace(kv, n_head, &need);
         if (!d_workspace || workspace_bytes < need) return TS_ERR_WORKSPACE;

@@ -918,19 +918,50 @@ def _split_kernel_name(cfg, n_cu=256):
     else:
         ctx = [cfg["ctx"] + 1] * cfg["batch"]
 
-    def chunk_for(target):
-        busy = lambda c: sum(-(-x // c) for x in ctx) * cfg["n_kv"]
-        hi = max(256, -(-max(ctx) // 64) * 64)
-        lo = min(hi, max(256, -(-sum(ctx) * cfg["n_kv"] // target)))
-        lo = -(-lo // 64) * 64
+    hd, n_kv, G = cfg["hd"], cfg["n_kv"], cfg["n_head"] // cfg["n_kv"]
+    stored = 64 if hd <= 64 else 128 if hd <= 128 else 256
+    top, total, S = max(ctx), sum(ctx), len(ctx)
+    n_win, wmax = -(-(top - 1) // 64), {64: 16, 128: 8, 256: 4}[stored]
+    if 4 < n_win <= wmax and S * n_kv * -(-G // 8) <= n_cu:
+        return "decode_split_kernel"
+    halves = -(-G // 4)
+    heads = 1.0 if halves <= 1 else 1.5 if halves == 2 else 2.5
+    cost = {  # fixed, per round, positions per round, workgroups at once, streams
+        1: ((5.0 if halves <= 1 else 7.5 if halves == 2 else 13.0) + (2.5 if stored == 256 else 0.0), (1.4 if halves <= 1 else 1.8 if halves == 2 else 3.2) if stored == 64
+            else (1.75 if stored == 256 else 0.95) * heads, 512 if stored == 64 else 256, n_cu, n_kv),
+        0: (4.0, {64: 1.33, 128: 1.55, 256: 3.2}[stored] * (1.4 if G > 4 else 1.0), 256, 1.25 * n_cu,
+            n_kv * -(-G // 8)),
+    }
+    bytes_us = total * n_kv * (stored + 8) / 6.5e6
+    most = min(-(-top // 256), min(-(-top // 64), 2 * n_cu // n_kv + 2))
+
+    def even(target, streams):
+        busy = lambda c: sum(-(-x // c) for x in ctx) * streams
+        hi = max(256, -(-top // 64) * 64)
+        lo = -(-min(hi, max(256, -(-total * streams // target))) // 64) * 64
         c = lo
         while c < hi and busy(c) > target:
             c += 64
         return lo if busy(c) > target else c  # no chunk meets the target: the balanced one
 
-    stored = 64 if cfg["hd"] <= 64 else 128 if cfg["hd"] <= 128 else 256
-    gmax = 16 if stored <= 128 else 8  # decode_int_gmax (ts_internal.h)
-    g4 = cfg["n_head"] // cfg["n_kv"] <= gmax and chunk_for(n_cu - n_cu // 8) >= 1024
+    kinds = (1, 0) if G <= (16 if stored <= 128 else 8) else (0,)  # decode_int_gmax (ts_internal.h)
+    c4 = even(n_cu - n_cu // 8, n_kv)
+    tries, k = [(c4, 1) if kinds[0] and c4 >= 1024 else (even(2 * n_cu, cost[0][4]), 0)], 1
+    while k <= most:
+        tries += [(-(-(-(-top // k) + (4 if k > 1 else 0)) // 64) * 64, kind) for kind in kinds]
+        k = k + 1 if k == most else min(most, k + (1 if k < 8 else k // 4))
+    best, g4 = None, 0
+    for chunk, kind in tries:
+        fixed, rnd, span, at_once, streams = cost[kind]
+        splits = [-(-x // chunk) for x in ctx]
+        cus = 0.875 if min(splits) != max(splits) else 1.0
+        us = longest = fixed + rnd * -(-min(chunk, top) // span)
+        if sum(splits) * streams > cus * n_cu:
+            work = sum(splits) * streams * (fixed + 0.5 * rnd) + rnd * total * streams / span
+            us = max(us, work / (cus * at_once) + 0.5 * longest)
+        us = max(us, bytes_us + fixed) + (3.5 if max(splits) > 1 else 0.0)
+        if best is None or us < 0.98 * best:
+            best, g4 = us, kind
     return "decode_split4_kernel" if g4 else "decode_split_kernel"
 
 
