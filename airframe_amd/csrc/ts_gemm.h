@@ -47,13 +47,18 @@ struct GemmTiles {
 };
 // f16 index inside tile row r of slot s (8 k).
 __device__ inline int tile_slot(int r, int s) { return 8 * (s ^ ((r >> 2) & 3)); }
+// Chunk c holds k 0-15 and 32-47 of its 64 (c even) or the other half, so that the k-steps of two
+// chunks are those of the slice loop (k 8q.. and 32 + 8q.. together) and the sums have the same
+// bits; slot s of a chunk starts tile_k(s) behind tile_chunk(c).
+__device__ inline size_t tile_chunk(int c) { return (size_t)(c >> 1) * 64 + (c & 1) * 16; }
+__device__ inline int tile_k(int s) { return 8 * (s & 1) + 32 * (s >> 1); }
 
 #define TS_SGB(mask, n) __builtin_amdgcn_sched_group_barrier(mask, n, 0)
 constexpr int kValu = 2, kMfma = 8, kVmemRead = 0x20, kDsRead = 0x100, kDsWrite = 0x200;
 
 // 64 rows x 256 columns over nch chunks of kTK, 256 threads: wave w accumulates rows 32 rb + ..,
 // columns 64 w + 32 cb + .. in acc[rb][cb].  Staging thread tid owns slot tid % 4 of x row tid / 4
-// and of weight rows tid / 4 + 64 i: xs / ws[i] point at it in chunk 0 (a row past the tile's last
+// and of weight rows tid / 4 + 64 i: xs / ws[i] point at its k (tile_k) of chunk 0 (a row past the tile's last
 // one points at any valid row: what it adds up to is not used).  xwrap: x has xwrap chunks and
 // weight chunk c multiplies x chunk c mod xwrap (nch = 2 xwrap: rows of two weight planes, hi
 // then lo, against the same x; nch = xwrap: one plane).
@@ -67,8 +72,10 @@ constexpr int kValu = 2, kMfma = 8, kVmemRead = 0x20, kDsRead = 0x100, kDsWrite 
 // between the matrix instructions of the same wave (two waves per SIMD do not cover for each
 // other between barriers).  Nothing in the loop is conditional (a skipped load would make every
 // wait for memory a wait for all of it): past the end the last chunk is loaded and stored again.
-// 2048 x 6144 outputs, 2560 long: 198 us with the weight rows loaded into the operands, 164 now
-// (785 TFLOP/s executed; all CUs together reach about 1.1 PFLOP/s on f16 matrix instructions).
+// 2048 x 6144 outputs, 2560 long: 198 us with the weight rows loaded into the operands, 187 now;
+// 2048 x 2560, 4096 long: 199, 149 (all CUs together reach about 1.1 PFLOP/s on f16 matrix
+// instructions; chunks of 32 k in a row took 164 and 134, but add in another order, and a last bit
+// moves a key or value next to a code's edge).
 // LDS bounds it: per chunk 48 KB read at 128 and 24 KB written at 75 bytes a clock, ~710 clocks
 // against 512 of matrix work.  128-row tiles (8 waves, or 4 of 64 x 128) were slower.
 __device__ __forceinline__ void gemm_tile_core(GemmTiles &sm, const float *xs, const _Float16 *const (&ws)[4],
@@ -85,10 +92,11 @@ __device__ __forceinline__ void gemm_tile_core(GemmTiles &sm, const float *xs, c
     auto load = [&](Stage &g, int c) {
         c = min(c, nch - 1);
         const int cx = c >= xwrap ? c - xwrap : c;
-        g.x[0] = *reinterpret_cast<const float4 *>(xs + (size_t)cx * kTK);
-        g.x[1] = *reinterpret_cast<const float4 *>(xs + (size_t)cx * kTK + 4);
+        const size_t kx = tile_chunk(cx), kw = tile_chunk(c);
+        g.x[0] = *reinterpret_cast<const float4 *>(xs + kx);
+        g.x[1] = *reinterpret_cast<const float4 *>(xs + kx + 4);
 #pragma unroll
-        for (int i = 0; i < 4; i++) g.w[i] = *reinterpret_cast<const half8 *>(ws[i] + (size_t)c * kTK);
+        for (int i = 0; i < 4; i++) g.w[i] = *reinterpret_cast<const half8 *>(ws[i] + kw);
     };
     auto store_x = [&](int buf, const Stage &g) {
         const int at = tile_slot(si, sc);
@@ -107,14 +115,14 @@ __device__ __forceinline__ void gemm_tile_core(GemmTiles &sm, const float *xs, c
     auto fetch = [&](Ops &o, int buf, int q) {
 #pragma unroll
         for (int rb = 0; rb < 2; rb++) {
-            const int r = 32 * rb + j, at = tile_slot(r, 2 * q + hf);
+            const int r = 32 * rb + j, at = tile_slot(r, 2 * hf + q);
             o.ah[rb] = *reinterpret_cast<const half8 *>(&sm.hi[buf][r][at]);
             o.al[rb] = *reinterpret_cast<const half8 *>(&sm.lo[buf][r][at]);
         }
 #pragma unroll
         for (int cb = 0; cb < 2; cb++) {
             const int r = 64 * wave + 32 * cb + j;
-            o.b[cb] = *reinterpret_cast<const half8 *>(&sm.w[buf][r][tile_slot(r, 2 * q + hf)]);
+            o.b[cb] = *reinterpret_cast<const half8 *>(&sm.w[buf][r][tile_slot(r, 2 * hf + q)]);
         }
     };
     auto multiply = [&](const Ops &o) {

@@ -193,7 +193,7 @@ struct QkvPlan {
 QkvPlan qkv_plan(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok);
 // GGUF block weights (Q4_K, Q5_K, Q8_0, Q4_0, Q5_0) read in the loop, dim a multiple of 256: the split
 // form with partials in `part` (part_bytes > 0), or with many tiles the tile kernel without any.
-QkvPlan qkv_plan_kq(int ggml_type, int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok);
+QkvPlan qkv_plan_kq(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok);
 hipError_t launch_qkv_kq(const KvLayerView &L, const int32_t *d_len, const float *x, int dim, int n_tok,
                          int ggml_type, const void *wq, const void *wk, const void *wv, int n_head,
                          float *q_out, float *k_out, float *v_out, const float *rope, int rope_pairs,
@@ -209,7 +209,7 @@ struct ProjPlan {
     uint64_t part_bytes;
 };
 ProjPlan proj_plan(int M, int K, int N);
-ProjPlan proj_plan_kq(int ggml_type, int M, int K, int N);  // block weights, K a multiple of 256
+ProjPlan proj_plan_kq(int M, int K, int N);  // block weights, K a multiple of 256
 hipError_t launch_proj_kq(const float *a, int M, int K, int ggml_type, const void *w, int N, float *act,
                           float *stash, const ProjPlan &plan, float *part, hipStream_t st);
 hipError_t launch_proj(const float *a, int M, int K, const uint16_t *w, int N, float *act, float *stash,

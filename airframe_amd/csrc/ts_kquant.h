@@ -56,12 +56,12 @@ void kq_dispatch(int t, F f) {
         f(std::integral_constant<int, kGgmlQ4_0>{});
 }
 // Whether a projection of that many 32 x 256 tiles takes the 64-row tile loop over the whole
-// reduction (one round of half as many workgroups) instead of slices and partials.  Measured
-// either way on whole blocks of 100 to 600 tokens, 2048 to 4096 wide: Q4_K, Q5_K and Q4_0 lose
-// 0.78-0.99 of their speed below 256 tiles and gain 1.06-1.27 just above (300 tokens of 4096: 1.06,
-// 420 of 3072: 1.27); Q8_0 and Q5_0, whose slices decode more, gain 1.05-1.2 from 192 tiles on
-// and lose below 160.
-inline bool kq_tiles(int t, int tiles32) { return tiles32 >= (t == kGgmlQ8_0 || t == kGgmlQ5_0 ? 192 : 256); }
+// reduction (one round of half as many workgroups) instead of slices and partials: where the
+// slices would not split the reduction either, so that the sums keep their bits.  Measured either
+// way on whole blocks of 100 to 600 tokens, 2048 to 4096 wide: below 256 tiles Q4_K, Q5_K and Q4_0
+// lose 0.78-0.99 of their speed (Q8_0 and Q5_0 gain up to 1.2 from 192 on), just above all gain
+// (300 tokens of 4096: 1.01-1.3, 420 of 3072: 1.27-1.57).
+inline bool kq_tiles(int tiles32) { return tiles32 >= 256; }
 
 // LDS of the K-quant slice loop: x of one super-block (4 chunks of 64) as hi/lo, and the f32
 // sums of its 8 sub-blocks per row.

@@ -694,11 +694,11 @@ struct QkvGenericKq {
     ts::ProjPlan pq, pk;
     uint64_t part_bytes, kv_elems;
 };
-static QkvGenericKq qkv_generic_plan_kq(const ts_kv *kv, int32_t ggml_type, int32_t dim, int32_t n_tok, int32_t n_head) {
+static QkvGenericKq qkv_generic_plan_kq(const ts_kv *kv, int32_t dim, int32_t n_tok, int32_t n_head) {
     QkvGenericKq g;
     const int M = kv->d.n_seq * n_tok, hd = kv->d.head_dim;
-    g.pq = ts::proj_plan_kq(ggml_type, M, dim, n_head * hd);
-    g.pk = ts::proj_plan_kq(ggml_type, M, dim, kv->d.n_head_kv * hd);
+    g.pq = ts::proj_plan_kq(M, dim, n_head * hd);
+    g.pk = ts::proj_plan_kq(M, dim, kv->d.n_head_kv * hd);
     g.part_bytes = (std::max(g.pq.part_bytes, g.pk.part_bytes) + 255) / 256 * 256;
     g.kv_elems = (uint64_t)M * kv->d.n_head_kv * hd;
     return g;
@@ -711,9 +711,9 @@ int ts_qkv_gguf_workspace(const ts_kv *kv, int32_t ggml_type, int32_t dim, int32
     *bytes = 0;
     if (n_tok == 0) return TS_OK;
     if (qkv_fused(kv)) {
-        *bytes = ts::qkv_plan_kq(ggml_type, kv->d.n_seq, kv->d.n_head_kv, n_head, kv->d.head_dim, dim, n_tok).part_bytes;
+        *bytes = ts::qkv_plan_kq(kv->d.n_seq, kv->d.n_head_kv, n_head, kv->d.head_dim, dim, n_tok).part_bytes;
     } else {
-        const QkvGenericKq g = qkv_generic_plan_kq(kv, ggml_type, dim, n_tok, n_head);
+        const QkvGenericKq g = qkv_generic_plan_kq(kv, dim, n_tok, n_head);
         *bytes = g.part_bytes + 2 * g.kv_elems * sizeof(float);
     }
     return TS_OK;
@@ -736,7 +736,7 @@ int ts_qkv_append_gguf(ts_kv *kv, int32_t layer, const float *d_x, int32_t dim, 
     if (n_tok == 0) return TS_OK;
     const hipStream_t st = as_stream(stream);
     if (!qkv_fused(kv)) {
-        const QkvGenericKq g = qkv_generic_plan_kq(kv, ggml_type, dim, n_tok, n_head);
+        const QkvGenericKq g = qkv_generic_plan_kq(kv, dim, n_tok, n_head);
         const uint64_t need = g.part_bytes + (d_k ? 0 : 2 * g.kv_elems * sizeof(float));
         if (!d_workspace || workspace_bytes < need || !aligned16(d_workspace)) return TS_ERR_WORKSPACE;
         float *part = static_cast<float *>(d_workspace);
@@ -754,7 +754,7 @@ int ts_qkv_append_gguf(ts_kv *kv, int32_t layer, const float *d_x, int32_t dim, 
                                          rope->rope_dim / 2, n_tok / 32 + 2, st);
         return hip_status(e);
     }
-    const ts::QkvPlan plan = ts::qkv_plan_kq(ggml_type, kv->d.n_seq, kv->d.n_head_kv, n_head, kv->d.head_dim, dim, n_tok);
+    const ts::QkvPlan plan = ts::qkv_plan_kq(kv->d.n_seq, kv->d.n_head_kv, n_head, kv->d.head_dim, dim, n_tok);
     if (!d_workspace || workspace_bytes < plan.part_bytes || !aligned16(d_workspace)) return TS_ERR_WORKSPACE;
     return hip_status(ts::launch_qkv_kq(kv->layer(layer), kv->d_len, d_x, dim, n_tok, ggml_type, d_wq, d_wk, d_wv,
                                         n_head, d_q, d_k, d_v, rope->d_table, rope->rope_dim / 2, plan,
@@ -764,7 +764,7 @@ int ts_qkv_append_gguf(ts_kv *kv, int32_t layer, const float *d_x, int32_t dim, 
 int ts_attn_out_proj_gguf_workspace(int32_t ggml_type, int32_t n_tok, int32_t attn_dim, int32_t dim, uint64_t *bytes) {
     if (!bytes || n_tok < 0 || attn_dim <= 0 || attn_dim % 256 != 0 || dim <= 0) return TS_ERR_INVALID;
     if (!kq_type_ok(ggml_type)) return TS_ERR_UNSUPPORTED;
-    *bytes = n_tok > 0 ? ts::proj_plan_kq(ggml_type, n_tok, attn_dim, dim).part_bytes : 0;
+    *bytes = n_tok > 0 ? ts::proj_plan_kq(n_tok, attn_dim, dim).part_bytes : 0;
     return TS_OK;
 }
 
@@ -776,7 +776,7 @@ int ts_attn_out_proj_gguf(const float *d_attn, int32_t n_tok, int32_t attn_dim, 
         return TS_ERR_INVALID;
     if (!kq_type_ok(ggml_type)) return TS_ERR_UNSUPPORTED;
     if (n_tok == 0) return TS_OK;
-    const ts::ProjPlan plan = ts::proj_plan_kq(ggml_type, n_tok, attn_dim, dim);
+    const ts::ProjPlan plan = ts::proj_plan_kq(n_tok, attn_dim, dim);
     if (!d_workspace || workspace_bytes < plan.part_bytes || !aligned16(d_workspace)) return TS_ERR_WORKSPACE;
     return hip_status(ts::launch_proj_kq(d_attn, n_tok, attn_dim, ggml_type, d_wo, dim, d_act, d_stash, plan,
                                          static_cast<float *>(d_workspace), as_stream(stream)));

@@ -64,8 +64,8 @@ __global__ __launch_bounds__(T == 0 ? 256 : 512, 2) void proj_tile_kernel(ProjAr
         const int si = tid >> 2, sc = tid & 3;
         const _Float16 *ws[4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) ws[i] = p.w + (size_t)min(col0 + si + 64 * i, p.N - 1) * p.KW + 8 * sc;
-        gemm_tile_core(sm, p.a + (size_t)min(row0 + si, p.M - 1) * p.K + 8 * sc, ws, p.KW / kTK, p.K / kTK, tid, acc);
+        for (int i = 0; i < 4; i++) ws[i] = p.w + (size_t)min(col0 + si + 64 * i, p.N - 1) * p.KW + tile_k(sc);
+        gemm_tile_core(sm, p.a + (size_t)min(row0 + si, p.M - 1) * p.K + tile_k(sc), ws, p.KW / kTK, p.K / kTK, tid, acc);
     } else {
         floatx16 c[2];
         gemm_tile_blocks<T>(sm, p.a + (size_t)min(row0 + (tid >> 3), p.M - 1) * p.K + 8 * (tid & 7),
@@ -257,12 +257,12 @@ ProjPlan proj_plan(int M, int K, int N) {
     return p;
 }
 
-ProjPlan proj_plan_kq(int ggml_type, int M, int K, int N) {
+ProjPlan proj_plan_kq(int M, int K, int N) {
     ProjPlan p;
     p.CT = (N + kPT - 1) / kPT;
     p.RT = (M + 31) / 32;
     const int tiles = p.RT * p.CT;
-    if (kq_tiles(ggml_type, tiles)) {
+    if (kq_tiles(tiles)) {
         p.RT = (M + 63) / 64;
         p.kps = K;
         p.n_split = 1;

@@ -357,12 +357,12 @@ __global__ __launch_bounds__(T == 0 ? 256 : 512, 2) void qkv_tile_kernel(QkvArgs
     const RowTile us = t[si / kMT];
     int xr = us.live ? x_row(a, us, si % kMT) : -1;
     if (xr < 0) xr = x_row(a, t[0], a.n_tok == 1 ? 0 : t[0].lo - t[0].blk * kBlk);
-    const float *xs = a.x + (size_t)xr * a.dim + 8 * sc;
+    const float *xs = a.x + (size_t)xr * a.dim + (T == 0 ? tile_k(sc) : 8 * sc);
     floatx16 acc[2][CB];
     if constexpr (T == 0) {
         const _Float16 *ws[4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) ws[i] = w_row(a, ct, si + 64 * i) + 8 * sc;
+        for (int i = 0; i < 4; i++) ws[i] = w_row(a, ct, si + 64 * i) + tile_k(sc);
         gemm_tile_core(sm.x, xs, ws, a.wld / kTK, a.dim / kTK, tid, acc);
     } else {
         floatx16 c[2];
@@ -586,14 +586,14 @@ QkvPlan qkv_plan(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok) {
     return p;
 }
 
-QkvPlan qkv_plan_kq(int ggml_type, int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok) {
+QkvPlan qkv_plan_kq(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok) {
     QkvPlan p;
     const int hpt = 128 / hd;
     p.CT = (n_head * hd + kNT - 1) / kNT + (n_kv + hpt - 1) / hpt;
     p.big = false;
     p.RT = n_tok == 1 ? (n_seq + kMT - 1) / kMT : n_seq * (n_tok / kBlk + 2);
     const int tiles = p.RT * p.CT;
-    if (kq_tiles(ggml_type, tiles)) {
+    if (kq_tiles(tiles)) {
         p.big = true;
         p.RT = (p.RT + 1) / 2;
         p.kps = dim;
