@@ -63,6 +63,24 @@ void kq_dispatch(int t, F f) {
 // (300 tokens of 4096: 1.01-1.3, 420 of 3072: 1.27-1.57).
 inline bool kq_tiles(int tiles32) { return tiles32 >= 256; }
 
+// Slices of a reduction over K (a multiple of 256) for fewer tiles than that, and the bytes of
+// their partials: splits for about one workgroup per CU (256; 512 and 1024 measured no faster at
+// 32 rows of 4096 x 4096).
+constexpr int kKqMaxSplit = 16;
+struct KqSlices {
+    int kps, n_split;
+    uint64_t bytes;
+};
+inline KqSlices kq_slices(int tiles32, int K) {
+    const int want = std::min(kKqMaxSplit, std::max(1, (256 + tiles32 - 1) / tiles32));
+    const int nbat = K / 256, per = (nbat + want - 1) / want;
+    KqSlices s;
+    s.kps = per * 256;
+    s.n_split = (nbat + per - 1) / per;
+    s.bytes = (uint64_t)s.n_split * tiles32 * (32 * 256) * sizeof(float);
+    return s;
+}
+
 // LDS of the K-quant slice loop: x of one super-block (4 chunks of 64) as hi/lo, and the f32
 // sums of its 8 sub-blocks per row.
 struct KqTiles {

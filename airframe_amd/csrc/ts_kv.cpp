@@ -710,11 +710,15 @@ int ts_qkv_gguf_workspace(const ts_kv *kv, int32_t ggml_type, int32_t dim, int32
     if (!kq_type_ok(ggml_type)) return TS_ERR_UNSUPPORTED;
     *bytes = 0;
     if (n_tok == 0) return TS_OK;
+    // enough for any n_tok up to this one: the tile kernels of long prompts take no scratch, and a
+    // caller sizes its buffer by its longest chunk
+    const int S = kv->d.n_seq, hd = kv->d.head_dim, H = kv->d.n_head_kv;
     if (qkv_fused(kv)) {
-        *bytes = ts::qkv_plan_kq(kv->d.n_seq, kv->d.n_head_kv, n_head, kv->d.head_dim, dim, n_tok).part_bytes;
+        *bytes = ts::qkv_part_bytes_kq(S, H, n_head, hd, dim, n_tok);
     } else {
-        const QkvGenericKq g = qkv_generic_plan_kq(kv, dim, n_tok, n_head);
-        *bytes = g.part_bytes + 2 * g.kv_elems * sizeof(float);
+        const uint64_t part = std::max(ts::proj_part_bytes_kq(S * n_tok, dim, n_head * hd),
+                                       ts::proj_part_bytes_kq(S * n_tok, dim, H * hd));
+        *bytes = (part + 255) / 256 * 256 + 2 * qkv_generic_plan_kq(kv, dim, n_tok, n_head).kv_elems * sizeof(float);
     }
     return TS_OK;
 }
@@ -738,7 +742,7 @@ int ts_qkv_append_gguf(ts_kv *kv, int32_t layer, const float *d_x, int32_t dim, 
     if (!qkv_fused(kv)) {
         const QkvGenericKq g = qkv_generic_plan_kq(kv, dim, n_tok, n_head);
         const uint64_t need = g.part_bytes + (d_k ? 0 : 2 * g.kv_elems * sizeof(float));
-        if (!d_workspace || workspace_bytes < need || !aligned16(d_workspace)) return TS_ERR_WORKSPACE;
+        if (need > 0 && (!d_workspace || workspace_bytes < need || !aligned16(d_workspace))) return TS_ERR_WORKSPACE;
         float *part = static_cast<float *>(d_workspace);
         float *kb = d_k ? d_k : reinterpret_cast<float *>(static_cast<uint8_t *>(d_workspace) + g.part_bytes);
         float *vb = d_k ? d_v : kb + g.kv_elems;
@@ -755,7 +759,8 @@ int ts_qkv_append_gguf(ts_kv *kv, int32_t layer, const float *d_x, int32_t dim, 
         return hip_status(e);
     }
     const ts::QkvPlan plan = ts::qkv_plan_kq(kv->d.n_seq, kv->d.n_head_kv, n_head, kv->d.head_dim, dim, n_tok);
-    if (!d_workspace || workspace_bytes < plan.part_bytes || !aligned16(d_workspace)) return TS_ERR_WORKSPACE;
+    if (plan.part_bytes > 0 && (!d_workspace || workspace_bytes < plan.part_bytes || !aligned16(d_workspace)))
+        return TS_ERR_WORKSPACE;
     return hip_status(ts::launch_qkv_kq(kv->layer(layer), kv->d_len, d_x, dim, n_tok, ggml_type, d_wq, d_wk, d_wv,
                                         n_head, d_q, d_k, d_v, rope->d_table, rope->rope_dim / 2, plan,
                                         static_cast<float *>(d_workspace), st));
@@ -764,7 +769,7 @@ int ts_qkv_append_gguf(ts_kv *kv, int32_t layer, const float *d_x, int32_t dim, 
 int ts_attn_out_proj_gguf_workspace(int32_t ggml_type, int32_t n_tok, int32_t attn_dim, int32_t dim, uint64_t *bytes) {
     if (!bytes || n_tok < 0 || attn_dim <= 0 || attn_dim % 256 != 0 || dim <= 0) return TS_ERR_INVALID;
     if (!kq_type_ok(ggml_type)) return TS_ERR_UNSUPPORTED;
-    *bytes = n_tok > 0 ? ts::proj_plan_kq(n_tok, attn_dim, dim).part_bytes : 0;
+    *bytes = n_tok > 0 ? ts::proj_part_bytes_kq(n_tok, attn_dim, dim) : 0;  // (any rows up to n_tok)
     return TS_OK;
 }
 
@@ -777,7 +782,8 @@ int ts_attn_out_proj_gguf(const float *d_attn, int32_t n_tok, int32_t attn_dim, 
     if (!kq_type_ok(ggml_type)) return TS_ERR_UNSUPPORTED;
     if (n_tok == 0) return TS_OK;
     const ts::ProjPlan plan = ts::proj_plan_kq(n_tok, attn_dim, dim);
-    if (!d_workspace || workspace_bytes < plan.part_bytes || !aligned16(d_workspace)) return TS_ERR_WORKSPACE;
+    if (plan.part_bytes > 0 && (!d_workspace || workspace_bytes < plan.part_bytes || !aligned16(d_workspace)))
+        return TS_ERR_WORKSPACE;
     return hip_status(ts::launch_proj_kq(d_attn, n_tok, attn_dim, ggml_type, d_wo, dim, d_act, d_stash, plan,
                                          static_cast<float *>(d_workspace), as_stream(stream)));
 }

@@ -23,7 +23,7 @@ namespace ts {
 namespace {
 
 constexpr int kPT = 256;        // columns per tile
-constexpr int kMaxPSplit = 16;  // most splits of the reduction
+constexpr int kMaxPSplit = kKqMaxSplit;  // most splits of the reduction
 
 struct ProjArgs {
     const float *a;      // [M][K] attention output
@@ -269,20 +269,23 @@ ProjPlan proj_plan_kq(int M, int K, int N) {
         p.part_bytes = 0;
         return p;
     }
-    // splits for about one workgroup per CU (256): measured on config 3's decode shapes, 512
-    // and 1024 were no faster (the split count is capped at kMaxPSplit anyway)
-    const int want = tiles < 256 ? std::min(kMaxPSplit, std::max(1, (256 + tiles - 1) / tiles)) : 1;
-    const int nbat = K / 256;
-    const int per = (nbat + want - 1) / want;
-    p.kps = per * 256;
-    p.n_split = (nbat + per - 1) / per;
-    p.part_bytes = (uint64_t)p.n_split * tiles * 32 * kPT * sizeof(float);
+    const KqSlices s = kq_slices(tiles, K);
+    p.kps = s.kps;
+    p.n_split = s.n_split;
+    p.part_bytes = s.bytes;
     return p;
+}
+
+uint64_t proj_part_bytes_kq(int M, int K, int N) {
+    const int CT = (N + kPT - 1) / kPT, RT = (M + 31) / 32;
+    uint64_t most = 0;
+    for (int rt = 1; rt <= RT && !kq_tiles(rt * CT); rt++) most = std::max(most, kq_slices(rt * CT, K).bytes);
+    return most;
 }
 
 hipError_t launch_proj_kq(const float *a, int M, int K, int ggml_type, const void *w, int N, float *act,
                           float *stash, const ProjPlan &plan, float *part, hipStream_t st) {
-    if (K % 256 != 0 || M <= 0 || N <= 0 || !part || !kq_type(ggml_type)) return hipErrorInvalidValue;
+    if (K % 256 != 0 || M <= 0 || N <= 0 || (plan.part_bytes > 0 && !part) || !kq_type(ggml_type)) return hipErrorInvalidValue;
     ProjArgs p;
     p.a = a;
     p.w = nullptr;

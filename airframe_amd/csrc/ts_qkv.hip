@@ -37,7 +37,7 @@ namespace {
 constexpr int kMT = 32;     // rows per tile
 constexpr int kNT = 256;    // columns per tile
 constexpr int kTStr = 260;  // LDS row stride of the output tile (f32)
-constexpr int kMaxSplit = 16;  // most splits of the reduction over dim
+constexpr int kMaxSplit = kKqMaxSplit;  // most splits of the reduction over dim
 
 struct QkvArgs {
     KvLayerView L;
@@ -601,23 +601,30 @@ QkvPlan qkv_plan_kq(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok)
         p.part_bytes = 0;
         return p;
     }
-    // few tiles: dim split over workgroups
-    // splits for about one workgroup per CU (256): measured on config 3's decode shapes, 512
-    // and 1024 were no faster (the split count is capped at kMaxSplit anyway)
-    const int want = tiles < 256 ? std::min(kMaxSplit, std::max(1, (256 + tiles - 1) / tiles)) : 1;
-    const int nbat = dim / 256;
-    const int per = (nbat + want - 1) / want;
-    p.kps = per * 256;
-    p.n_split = (nbat + per - 1) / per;
-    p.part_bytes = (uint64_t)p.n_split * tiles * kMT * kNT * sizeof(float);
+    const KqSlices s = kq_slices(tiles, dim);
+    p.kps = s.kps;
+    p.n_split = s.n_split;
+    p.part_bytes = s.bytes;
     return p;
+}
+
+uint64_t qkv_part_bytes_kq(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok) {
+    uint64_t most = 0;
+    // (a token count sets the tiles through n_tok / kBlk alone, apart from one token's)
+    for (int t = 1; t <= n_tok; t = t == 1 ? 2 : t < kBlk ? kBlk : t + kBlk) {
+        const QkvPlan p = qkv_plan_kq(n_seq, n_kv, n_head, hd, dim, t);
+        if (t > 1 && p.big) break;
+        most = std::max(most, p.part_bytes);
+    }
+    return most;
 }
 
 hipError_t launch_qkv_kq(const KvLayerView &L, const int32_t *d_len, const float *x, int dim, int n_tok,
                          int ggml_type, const void *wq, const void *wk, const void *wv, int n_head,
                          float *q_out, float *k_out, float *v_out, const float *rope, int rope_pairs,
                          const QkvPlan &plan, float *part, hipStream_t st) {
-    if ((L.hd != 128 && L.hd != 64) || dim % 256 != 0 || !part || !kq_type(ggml_type)) return hipErrorInvalidValue;
+    if ((L.hd != 128 && L.hd != 64) || dim % 256 != 0 || (plan.part_bytes > 0 && !part) || !kq_type(ggml_type))
+        return hipErrorInvalidValue;
     QkvArgs a;
     a.L = L;
     a.len = d_len;

@@ -346,8 +346,9 @@ int ts_attn_out_proj_x2(const float *d_attn, int32_t n_tok, int32_t attn_dim, co
 
 /* ---- projections with GGUF block weights read at their own size --------------------------- */
 
-/* Bytes of scratch ts_qkv_append_gguf needs for this shape (ggml_type TS_GGML_Q4_K,
- * TS_GGML_Q5_K, TS_GGML_Q8_0, TS_GGML_Q4_0 or TS_GGML_Q5_0; dim a multiple of 256).  Host
+/* Bytes of scratch that cover ts_qkv_append_gguf for this shape with n_tok tokens or any fewer
+ * (ggml_type TS_GGML_Q4_K, TS_GGML_Q5_K, TS_GGML_Q8_0, TS_GGML_Q4_0 or TS_GGML_Q5_0; dim a
+ * multiple of 256), so that a buffer sized for the longest chunk serves the shorter ones.  Host
  * only. */
 int ts_qkv_gguf_workspace(const ts_kv *kv, int32_t ggml_type, int32_t dim, int32_t n_tok, int32_t n_head,
                           uint64_t *bytes);
@@ -360,14 +361,16 @@ int ts_qkv_gguf_workspace(const ts_kv *kv, int32_t ggml_type, int32_t dim, int32
  * [n_head*head_dim] rows of dim elements, d_wk, d_wv: [n_head_kv*head_dim] rows, all 16-byte
  * aligned (the blocks of one type for all three); dim a multiple of 256.  Results agree with the
  * f32-weight dot to f32 rounding (x is split hi + lo in f16, |x| < 65504, as in ts_qkv_append).
- * Any other type is TS_ERR_UNSUPPORTED: convert it once with ts_weights_to_f16x2.  The
- * workspace is always needed (ts_qkv_gguf_workspace). */
+ * Any other type is TS_ERR_UNSUPPORTED: convert it once with ts_weights_to_f16x2.  d_workspace:
+ * ts_qkv_gguf_workspace bytes, 16-byte aligned (not looked at, and may be NULL, in a call that
+ * splits no reduction and stages no K and V: the long chunks, whose tiles fill the chip). */
 int ts_qkv_append_gguf(ts_kv *kv, int32_t layer, const float *d_x, int32_t dim, int32_t n_tok, int32_t ggml_type,
                        const void *d_wq, const void *d_wk, const void *d_wv, int32_t n_head, const ts_rope *rope,
                        float *d_q, float *d_k, float *d_v, void *d_workspace, uint64_t workspace_bytes,
                        void *stream);
 
-/* Bytes of scratch ts_attn_out_proj_gguf needs (attn_dim a multiple of 256).  Host only. */
+/* Bytes of scratch that cover ts_attn_out_proj_gguf for n_tok rows or any fewer (attn_dim a
+ * multiple of 256; the workspace as in ts_qkv_append_gguf).  Host only. */
 int ts_attn_out_proj_gguf_workspace(int32_t ggml_type, int32_t n_tok, int32_t attn_dim, int32_t dim,
                                     uint64_t *bytes);
 
