@@ -10,7 +10,9 @@
 // result is complete in one kernel and deterministic.
 //
 // x is used as it is (f32, no hi/lo split); products with f16 weights and with the integer codes
-// are fused multiply-adds into f32, block scales are applied to the sum over the block.
+// are fused multiply-adds into f32, block scales are applied to the sum over the block.  The codes
+// of Q4_0 and Q5_0 are taken signed (n - 8, n - 16, exact): with n alone and 8 or 16 times the sum
+// of x subtracted, the two cancel and leave 1.5 to 2.4 times the error of the matrix-core slices.
 //
 // One row of Q4_K: 3072 -> 5120 (QKV) 11.6 + 6.2 us (slices + sum and append) -> 7.3 + 3.5 (this +
 // append), 3072 -> 3072 with the residual 8.8 + 3.2 -> 5.8; launch and the x -> LDS -> sum chain
@@ -80,9 +82,10 @@ __device__ __forceinline__ void gemv_load(GemvRaw<T> &r, const uint8_t *at, size
     }
 }
 
-// The share's weights as f32 integers (K formats and blocks) or values (f16), w[plane][e] at k
-// gemv_k(p, e), and the factors that make the sum over them a result: with s0, s1 the sums over
-// elements 0-15 and 16-31 and t0, t1 the sums of x over the same, a0 s0 + a1 s1 + c0 t0 + c1 t1.
+// The share's weights as f32 integers (the codes, signed except in the K formats), w[e] at k
+// gemv_k(p, e), and the factors that make the sum over them a result: a0 times it; in the K formats,
+// with s0, s1 the sums over elements 0-15 and 16-31 and t0, t1 the sums of x over the same,
+// a0 s0 + a1 s1 + c0 t0 + c1 t1.
 template <int T>
 struct GemvWeights {
     float w[32];
@@ -125,9 +128,8 @@ __device__ __forceinline__ void gemv_decode(GemvWeights<T> &g, const GemvRaw<T> 
         };
         const uint32_t dbits = odd ? r.w[0] >> 16 : r.w[0] & 0xFFFFu;
         const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)dbits);
-        g.a0 = g.a1 = d;
+        g.a0 = d;
         if constexpr (T == kGgmlQ8_0) {
-            g.c0 = g.c1 = 0.0f;
 #pragma unroll
             for (int i = 0; i < 8; i++) {
                 const uint32_t v = word(i);
@@ -135,7 +137,7 @@ __device__ __forceinline__ void gemv_decode(GemvWeights<T> &g, const GemvRaw<T> 
                 for (int b = 0; b < 4; b++) g.w[4 * i + b] = (float)(int8_t)(v >> (8 * b));
             }
         } else {
-            g.c0 = g.c1 = d * (T == kGgmlQ5_0 ? -16.0f : -8.0f);
+            constexpr float mid = T == kGgmlQ5_0 ? 16.0f : 8.0f;
             const uint32_t qh = T == kGgmlQ5_0 ? word(0) : 0u;
             constexpr int first = T == kGgmlQ5_0 ? 1 : 0;
 #pragma unroll
@@ -149,8 +151,8 @@ __device__ __forceinline__ void gemv_decode(GemvWeights<T> &g, const GemvRaw<T> 
                 }
 #pragma unroll
                 for (int b = 0; b < 4; b++) {
-                    g.w[4 * i + b] = ub(lo, b);
-                    g.w[16 + 4 * i + b] = ub(hi, b);
+                    g.w[4 * i + b] = ub(lo, b) - mid;
+                    g.w[16 + 4 * i + b] = ub(hi, b) - mid;
                 }
             }
         }
@@ -221,15 +223,21 @@ __device__ __forceinline__ void gemv_rows(float *sx, float *red, const float *x,
                             }
                     }
             } else {
+                constexpr bool K = T == kGgmlQ4K || T == kGgmlQ5K;
                 GemvWeights<T> g[R];
 #pragma unroll
                 for (int r = 0; r < R; r++) gemv_decode<T>(g[r], raw[r], p);
 #pragma unroll
                 for (int m = 0; m < MB; m++) {
-                    float s[R][2];
+                    // K formats: a sum per sub-block; the others: four chains of eight k (two of sixteen
+                    // have a tenth more error)
+                    constexpr int NS = K ? 2 : 4;
+                    float s[R][NS];
                     float t[2] = {0.0f, 0.0f};
 #pragma unroll
-                    for (int r = 0; r < R; r++) s[r][0] = s[r][1] = 0.0f;
+                    for (int r = 0; r < R; r++)
+#pragma unroll
+                        for (int c = 0; c < NS; c++) s[r][c] = 0.0f;
 #pragma unroll
                     for (int i = 0; i < 8; i++) {
                         const float4 u = *reinterpret_cast<const float4 *>(xb + m * seg + gemv_k<T>(p, 4 * i));
@@ -237,14 +245,20 @@ __device__ __forceinline__ void gemv_rows(float *sx, float *red, const float *x,
 #pragma unroll
                         for (int r = 0; r < R; r++)
 #pragma unroll
-                            for (int e = 0; e < 4; e++) s[r][i >> 2] = __builtin_fmaf(g[r].w[4 * i + e], xv[e], s[r][i >> 2]);
-                        if constexpr (T != kGgmlQ8_0) t[i >> 2] = t[i >> 2] + ((u.x + u.y) + (u.z + u.w));
+                            for (int e = 0; e < 4; e++) {
+                                float &sum = s[r][K ? i >> 2 : e];
+                                sum = __builtin_fmaf(g[r].w[4 * i + e], xv[e], sum);
+                            }
+                        if constexpr (K) t[i >> 2] = t[i >> 2] + ((u.x + u.y) + (u.z + u.w));
                     }
 #pragma unroll
                     for (int r = 0; r < R; r++) {
-                        float v = __builtin_fmaf(g[r].a1, s[r][1], g[r].a0 * s[r][0]);
-                        if constexpr (T != kGgmlQ8_0) v = __builtin_fmaf(g[r].c1, t[1], __builtin_fmaf(g[r].c0, t[0], v));
-                        acc[r][m] = acc[r][m] + v;
+                        if constexpr (K) {
+                            const float v = __builtin_fmaf(g[r].a1, s[r][1], g[r].a0 * s[r][0]);
+                            acc[r][m] = acc[r][m] + __builtin_fmaf(g[r].c1, t[1], __builtin_fmaf(g[r].c0, t[0], v));
+                        } else {
+                            acc[r][m] = __builtin_fmaf(g[r].a0, (s[r][0] + s[r][1]) + (s[r][NS - 2] + s[r][NS - 1]), acc[r][m]);
+                        }
                     }
                 }
             }

@@ -1,0 +1,58 @@
+"""Decode of one or two rows is no less precise than the matrix-core slices that more rows take: the
+vector-unit kernels' error against 64 bits next to the slices' on the same rows and weights (2-norm
+over 2 x 2048 results, so that either is known to about 2%), for every weight form."""
+import numpy as np
+import pytest
+import torch
+
+from airframe_amd import weights
+from airframe_amd.kv_cache import attn_out_proj, attn_out_proj_gguf
+from oracle import oracle
+from tests.gpu_util import dev, say
+from tests.test_gpu_weights import random_blob
+
+pytestmark = pytest.mark.gpu
+
+BLOCKS = {"q4_0": weights.Q4_0, "q5_0": weights.Q5_0, "q8_0": weights.Q8_0, "q4_k": weights.Q4_K, "q5_k": weights.Q5_K}
+
+
+def project(form, a, w, dim):
+    """The raw product of the rows of a."""
+    act = torch.zeros((a.shape[0], dim), dtype=torch.float32, device="cuda")
+    stash = torch.empty_like(act)
+    if form in BLOCKS:
+        attn_out_proj_gguf(a, BLOCKS[form], w, dim, act, stash=stash)
+    else:
+        attn_out_proj(a, w, act, stash=stash, planes=2 if form == "f16x2" else 1)
+    torch.cuda.synchronize()
+    return stash.cpu().numpy().astype(np.float64)
+
+
+@pytest.mark.parametrize("form", ["q4_0", "q5_0"])
+@pytest.mark.parametrize("n_tok", [1, 2])
+@pytest.mark.parametrize("attn_dim", [512, 4096, 8192])
+def test_rows_error(gpu, form, n_tok, attn_dim):
+    say(f"gemv error form={form} n_tok={n_tok} attn_dim={attn_dim}")
+    rng = np.random.default_rng(attn_dim + n_tok)
+    dim = 2048
+    if form in BLOCKS:
+        blob = random_blob(rng, BLOCKS[form], dim, attn_dim)
+        w = dev(blob)
+        wf = oracle.dequant(BLOCKS[form], blob, dim * attn_dim).reshape(dim, attn_dim).astype(np.float64)
+    else:
+        full = (rng.standard_normal((dim, attn_dim)) * 0.02).astype(np.float32)
+        hi = full.astype(np.float16)
+        lo = (full - hi.astype(np.float32)).astype(np.float16)
+        w = dev(np.concatenate([hi, lo], 1) if form == "f16x2" else hi)
+        wf = hi.astype(np.float64) + (lo.astype(np.float64) if form == "f16x2" else 0.0)
+    a = rng.standard_normal((2, attn_dim)).astype(np.float32)
+    ref = a.astype(np.float64) @ wf.T
+
+    def error(got):
+        return np.linalg.norm(got - ref) / np.linalg.norm(ref)
+
+    rows = np.concatenate([project(form, dev(a[i:i + n_tok]), w, dim) for i in range(0, 2, n_tok)])
+    gemv, slices = error(rows), error(project(form, dev(np.concatenate([a, a])), w, dim)[:2])
+    say(f"  error {gemv:.3e}, slices {slices:.3e}")
+    # (1.06: three times the 2%)
+    assert gemv <= 1.06 * slices
