@@ -28,7 +28,7 @@ def project(form, a, w, dim):
     return stash.cpu().numpy().astype(np.float64)
 
 
-@pytest.mark.parametrize("form", ["q4_0", "q5_0"])
+@pytest.mark.parametrize("form", ["f16", "f16x2", "q4_0", "q5_0", "q8_0", "q4_k", "q5_k"])
 @pytest.mark.parametrize("n_tok", [1, 2])
 @pytest.mark.parametrize("attn_dim", [512, 4096, 8192])
 def test_rows_error(gpu, form, n_tok, attn_dim):
