@@ -313,8 +313,16 @@ __device__ __forceinline__ void gemv_rows(float *sx, float *red, const float *x,
 inline int gemv_mb(int M) { return M <= 1 ? 1 : 2; }
 // Weight rows per lane: two share the x reads once there is more than one row of x.
 __host__ __device__ constexpr int gemv_r(int mb) { return mb == 1 ? 1 : 2; }
-// Whether M rows of K take these kernels.
-inline bool gemv_fits(int M, int K) { return M <= kGemvRows && K % 256 == 0; }
+// Whether M rows of K take these kernels for N weight rows of form t.  Two rows of more than 6144 pass
+// LDS in pieces that the slices do without: in us, slices then these, 2 x 12288 -> 4096: Q4_K 19.4,
+// 22.4, Q5_K 22.0, 24.1, f16 28.5, 30.7; 2 x 8192 -> 10240 in two planes 82, 102.  With 8192 weight
+// rows to share x they win all the same (8192 -> 8192: Q4_K 22.9, 20.4, f16 36.6, 33.6), and always
+// where the slices are bound by decoding (Q8_0, Q4_0, Q5_0: 0.35 to 0.97 of their time).
+inline bool gemv_fits(int t, int M, int K, int N) {
+    if (M > kGemvRows || K % 256 != 0) return false;
+    if (M == 1 || K <= 6144) return true;
+    return t == kGgmlQ8_0 || t == kGgmlQ4_0 || t == kGgmlQ5_0 || (t != kGemvF16x2 && N >= 8192);
+}
 inline size_t gemv_lds(int mb, int K) { return std::min<size_t>((size_t)mb * K * 4, kGemvLds); }
 
 // f(integral_constant<int, T>, integral_constant<int, MB>) for f16 rows of 1 or 2 planes (type 0 or

@@ -303,7 +303,7 @@ hipError_t launch_proj_kq(const float *a, int M, int K, int ggml_type, const voi
     p.kps = plan.kps;
     p.n_split = plan.n_split;
     p.n_wg = plan.RT * plan.CT * plan.n_split;
-    if (gemv_fits(M, K) && plan.part_bytes > 0) {
+    if (gemv_fits(ggml_type, M, K, N) && plan.part_bytes > 0) {
         proj_gemv(ggml_type, p, st);
         return hipGetLastError();
     }
@@ -342,7 +342,7 @@ hipError_t launch_proj(const float *a, int M, int K, const uint16_t *w, int N, f
     const int grid = (p.n_wg + 7) / 8 * 8;
     if (plan.n_split == 1) {
         proj_tile_kernel<0><<<grid, 256, 0, st>>>(p);
-    } else if (gemv_fits(M, K)) {
+    } else if (gemv_fits(planes == 2 ? kGemvF16x2 : kGemvF16, M, K, N)) {
         proj_gemv(planes == 2 ? kGemvF16x2 : kGemvF16, p, st);
     } else {
         proj_split_kernel<<<grid, 256, 0, st>>>(p);

@@ -652,7 +652,8 @@ hipError_t launch_qkv_kq(const KvLayerView &L, const int32_t *d_len, const float
     a.kps = plan.kps;
     a.n_split = plan.n_split;
     a.n_wg = plan.RT * plan.CT * plan.n_split;
-    if (n_tok == 1 && gemv_fits(L.S, dim) && !plan.big) return qkv_gemv(ggml_type, a, part, st);
+    const int rows = (n_head + 2 * L.H) * L.hd;
+    if (n_tok == 1 && gemv_fits(ggml_type, L.S, dim, rows) && !plan.big) return qkv_gemv(ggml_type, a, part, st);
     const int grid = (a.n_wg + 7) / 8 * 8;
     kq_dispatch(ggml_type, [&](auto tc) {
         constexpr int T = decltype(tc)::value;
@@ -702,8 +703,8 @@ hipError_t launch_qkv(const KvLayerView &L, const int32_t *d_len, const float *x
     a.n_split = plan.n_split;
     a.n_wg = plan.RT * plan.CT * plan.n_split;
     // (the split plans' scratch is at least 256 floats for every K and V column of 32 rows)
-    if (n_tok == 1 && gemv_fits(L.S, dim) && !plan.big)
-        return qkv_gemv(planes == 2 ? kGemvF16x2 : kGemvF16, a, part, st);
+    const int form = planes == 2 ? kGemvF16x2 : kGemvF16, rows = (n_head + 2 * L.H) * L.hd;
+    if (n_tok == 1 && gemv_fits(form, L.S, dim, rows) && !plan.big) return qkv_gemv(form, a, part, st);
     const int grid = (a.n_wg + 7) / 8 * 8;
     if (plan.big) {
         qkv_tile_kernel<0><<<grid, 256, 0, st>>>(a);
