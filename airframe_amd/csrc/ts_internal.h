@@ -134,6 +134,11 @@ struct ts_rope {
 
 namespace ts {
 
+// Whether two ranges of na and nb f32 share memory (null: empty).
+inline bool overlap(const float *a, uint64_t na, const float *b, uint64_t nb) {
+    return a && b && a < b + nb && b < a + na;
+}
+
 // Kernel launchers (defined in the .hip files).  All return hipError_t of the launch.
 hipError_t launch_quantize_rows(const KvLayerView &L, const float *k, const float *v,
                                 const int32_t *d_start, int32_t fixed_start, int32_t count,
@@ -189,11 +194,14 @@ struct QkvPlan {
     int kps, n_split;     // reduction length per split, splits
     bool big;             // one workgroup per 64-row tile over all of dim (else split)
     uint64_t part_bytes;  // scratch for the split partials (0 without a split)
+    // An output shares memory with x (a caller that reuses x for q, say): the partials, which no
+    // output is written before, instead of the kernels that read x while they write.
+    bool in_place = false;
 };
 QkvPlan qkv_plan(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok);
 // GGUF block weights (Q4_K, Q5_K, Q8_0, Q4_0, Q5_0) read in the loop, dim a multiple of 256: the split
 // form with partials in `part` (part_bytes > 0), or with many tiles the tile kernel without any.
-QkvPlan qkv_plan_kq(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok);
+QkvPlan qkv_plan_kq(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok, bool in_place = false);
 // The most part_bytes of qkv_plan_kq for 1 to n_tok tokens.
 uint64_t qkv_part_bytes_kq(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok);
 hipError_t launch_qkv_kq(const KvLayerView &L, const int32_t *d_len, const float *x, int dim, int n_tok,
@@ -209,9 +217,10 @@ hipError_t launch_qkv(const KvLayerView &L, const int32_t *d_len, const float *x
 struct ProjPlan {
     int RT, CT, kps, n_split;
     uint64_t part_bytes;
+    bool in_place = false;  // act or stash shares memory with the input (as QkvPlan)
 };
 ProjPlan proj_plan(int M, int K, int N);
-ProjPlan proj_plan_kq(int M, int K, int N);  // block weights, K a multiple of 256
+ProjPlan proj_plan_kq(int M, int K, int N, bool in_place = false);  // block weights, K a multiple of 256
 uint64_t proj_part_bytes_kq(int M, int K, int N);  // the most part_bytes of it for 1 to M rows
 hipError_t launch_proj_kq(const float *a, int M, int K, int ggml_type, const void *w, int N, float *act,
                           float *stash, const ProjPlan &plan, float *part, hipStream_t st);

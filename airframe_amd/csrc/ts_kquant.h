@@ -63,9 +63,9 @@ void kq_dispatch(int t, F f) {
 // (300 tokens of 4096: 1.01-1.3, 420 of 3072: 1.27-1.57).
 inline bool kq_tiles(int tiles32) { return tiles32 >= 256; }
 
-// Slices of a reduction over K (a multiple of 256) for fewer tiles than that, and the bytes of
-// their partials: splits for about one workgroup per CU (256; 512 and 1024 measured no faster at
-// 32 rows of 4096 x 4096).
+// Slices of a reduction over K (a multiple of 256) for fewer tiles than that (one slice for more),
+// and the bytes of their partials: splits for about one workgroup per CU (256; 512 and 1024 measured
+// no faster at 32 rows of 4096 x 4096).
 constexpr int kKqMaxSplit = 16;
 struct KqSlices {
     int kps, n_split;

@@ -592,6 +592,14 @@ static bool qkv_shape_ok(const ts_kv *kv, int32_t dim, int32_t n_tok, int32_t n_
 // is the dot) and then the append kernel on the projected K and V.
 static bool qkv_fused(const ts_kv *kv) { return kv->d.head_dim == 128 || kv->d.head_dim == 64; }
 
+// Whether q, k or v of a QKV call shares memory with x.
+static bool qkv_in_place(const ts_kv *kv, const float *d_x, int32_t dim, int32_t n_tok, int32_t n_head, const float *d_q,
+                         const float *d_k, const float *d_v) {
+    const uint64_t M = (uint64_t)kv->d.n_seq * n_tok, nq = M * n_head * kv->d.head_dim,
+                   nk = M * kv->d.n_head_kv * kv->d.head_dim;
+    return ts::overlap(d_x, M * dim, d_q, nq) || ts::overlap(d_x, M * dim, d_k, nk) || ts::overlap(d_x, M * dim, d_v, nk);
+}
+
 struct QkvGeneric {
     ts::ProjPlan pq, pk;
     uint64_t part_bytes;  // split partials, shared by the three projections (256-aligned)
@@ -660,7 +668,8 @@ static int qkv_append_planes(ts_kv *kv, int32_t layer, const float *d_x, int32_t
                                          rope->rope_dim / 2, n_tok / 32 + 2, st);
         return hip_status(e);
     }
-    const ts::QkvPlan plan = ts::qkv_plan(kv->d.n_seq, kv->d.n_head_kv, n_head, kv->d.head_dim, planes * dim, n_tok);
+    ts::QkvPlan plan = ts::qkv_plan(kv->d.n_seq, kv->d.n_head_kv, n_head, kv->d.head_dim, planes * dim, n_tok);
+    plan.in_place = qkv_in_place(kv, d_x, dim, n_tok, n_head, d_q, d_k, d_v);
     if (plan.part_bytes > 0 && (!d_workspace || workspace_bytes < plan.part_bytes || !aligned16(d_workspace)))
         return TS_ERR_WORKSPACE;
     return hip_status(ts::launch_qkv(kv->layer(layer), kv->d_len, d_x, dim, n_tok, d_wq, d_wk, d_wv,
@@ -758,12 +767,20 @@ int ts_qkv_append_gguf(ts_kv *kv, int32_t layer, const float *d_x, int32_t dim, 
                                          rope->rope_dim / 2, n_tok / 32 + 2, st);
         return hip_status(e);
     }
-    const ts::QkvPlan plan = ts::qkv_plan_kq(kv->d.n_seq, kv->d.n_head_kv, n_head, kv->d.head_dim, dim, n_tok);
+    const ts::QkvPlan plan = ts::qkv_plan_kq(kv->d.n_seq, kv->d.n_head_kv, n_head, kv->d.head_dim, dim, n_tok,
+                                             qkv_in_place(kv, d_x, dim, n_tok, n_head, d_q, d_k, d_v));
     if (plan.part_bytes > 0 && (!d_workspace || workspace_bytes < plan.part_bytes || !aligned16(d_workspace)))
         return TS_ERR_WORKSPACE;
     return hip_status(ts::launch_qkv_kq(kv->layer(layer), kv->d_len, d_x, dim, n_tok, ggml_type, d_wq, d_wk, d_wv,
                                         n_head, d_q, d_k, d_v, rope->d_table, rope->rope_dim / 2, plan,
                                         static_cast<float *>(d_workspace), st));
+}
+
+// Whether act or the stash of an output projection shares memory with its input.
+static bool proj_in_place(const float *d_attn, int32_t n_tok, int32_t attn_dim, int32_t dim, const float *d_act,
+                          const float *d_stash) {
+    const uint64_t in = (uint64_t)n_tok * attn_dim, out = (uint64_t)n_tok * dim;
+    return ts::overlap(d_attn, in, d_act, out) || ts::overlap(d_attn, in, d_stash, out);
 }
 
 int ts_attn_out_proj_gguf_workspace(int32_t ggml_type, int32_t n_tok, int32_t attn_dim, int32_t dim, uint64_t *bytes) {
@@ -781,7 +798,8 @@ int ts_attn_out_proj_gguf(const float *d_attn, int32_t n_tok, int32_t attn_dim, 
         return TS_ERR_INVALID;
     if (!kq_type_ok(ggml_type)) return TS_ERR_UNSUPPORTED;
     if (n_tok == 0) return TS_OK;
-    const ts::ProjPlan plan = ts::proj_plan_kq(n_tok, attn_dim, dim);
+    const ts::ProjPlan plan =
+        ts::proj_plan_kq(n_tok, attn_dim, dim, proj_in_place(d_attn, n_tok, attn_dim, dim, d_act, d_stash));
     if (plan.part_bytes > 0 && (!d_workspace || workspace_bytes < plan.part_bytes || !aligned16(d_workspace)))
         return TS_ERR_WORKSPACE;
     return hip_status(ts::launch_proj_kq(d_attn, n_tok, attn_dim, ggml_type, d_wo, dim, d_act, d_stash, plan,
@@ -803,7 +821,8 @@ static int out_proj_planes(const float *d_attn, int32_t n_tok, int32_t attn_dim,
         !aligned16(d_attn) || !aligned16(d_wo) || !aligned16(d_act) || !aligned16(d_stash))
         return TS_ERR_INVALID;
     if (n_tok == 0) return TS_OK;
-    const ts::ProjPlan plan = ts::proj_plan(n_tok, planes * attn_dim, dim);
+    ts::ProjPlan plan = ts::proj_plan(n_tok, planes * attn_dim, dim);
+    plan.in_place = proj_in_place(d_attn, n_tok, attn_dim, dim, d_act, d_stash);
     if (plan.part_bytes > 0 && (!d_workspace || workspace_bytes < plan.part_bytes || !aligned16(d_workspace)))
         return TS_ERR_WORKSPACE;
     return hip_status(ts::launch_proj(d_attn, n_tok, attn_dim, d_wo, dim, d_act, d_stash, plan,

@@ -257,12 +257,13 @@ ProjPlan proj_plan(int M, int K, int N) {
     return p;
 }
 
-ProjPlan proj_plan_kq(int M, int K, int N) {
+ProjPlan proj_plan_kq(int M, int K, int N, bool in_place) {
     ProjPlan p;
+    p.in_place = in_place;
     p.CT = (N + kPT - 1) / kPT;
     p.RT = (M + 31) / 32;
     const int tiles = p.RT * p.CT;
-    if (kq_tiles(tiles)) {
+    if (kq_tiles(tiles) && !in_place) {
         p.RT = (M + 63) / 64;
         p.kps = K;
         p.n_split = 1;
@@ -285,7 +286,8 @@ uint64_t proj_part_bytes_kq(int M, int K, int N) {
 
 hipError_t launch_proj_kq(const float *a, int M, int K, int ggml_type, const void *w, int N, float *act,
                           float *stash, const ProjPlan &plan, float *part, hipStream_t st) {
-    if (K % 256 != 0 || M <= 0 || N <= 0 || (plan.part_bytes > 0 && !part) || !kq_type(ggml_type)) return hipErrorInvalidValue;
+    if (K % 256 != 0 || M <= 0 || N <= 0 || (plan.part_bytes > 0 && !part) || !kq_type(ggml_type))
+        return hipErrorInvalidValue;
     ProjArgs p;
     p.a = a;
     p.w = nullptr;
@@ -303,7 +305,7 @@ hipError_t launch_proj_kq(const float *a, int M, int K, int ggml_type, const voi
     p.kps = plan.kps;
     p.n_split = plan.n_split;
     p.n_wg = plan.RT * plan.CT * plan.n_split;
-    if (gemv_fits(ggml_type, M, K, N) && plan.part_bytes > 0) {
+    if (gemv_fits(ggml_type, M, K, N) && plan.part_bytes > 0 && !plan.in_place) {
         proj_gemv(ggml_type, p, st);
         return hipGetLastError();
     }
@@ -342,7 +344,7 @@ hipError_t launch_proj(const float *a, int M, int K, const uint16_t *w, int N, f
     const int grid = (p.n_wg + 7) / 8 * 8;
     if (plan.n_split == 1) {
         proj_tile_kernel<0><<<grid, 256, 0, st>>>(p);
-    } else if (gemv_fits(planes == 2 ? kGemvF16x2 : kGemvF16, M, K, N)) {
+    } else if (gemv_fits(planes == 2 ? kGemvF16x2 : kGemvF16, M, K, N) && !plan.in_place) {
         proj_gemv(planes == 2 ? kGemvF16x2 : kGemvF16, p, st);
     } else {
         proj_split_kernel<<<grid, 256, 0, st>>>(p);

@@ -586,14 +586,15 @@ QkvPlan qkv_plan(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok) {
     return p;
 }
 
-QkvPlan qkv_plan_kq(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok) {
+QkvPlan qkv_plan_kq(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok, bool in_place) {
     QkvPlan p;
+    p.in_place = in_place;
     const int hpt = 128 / hd;
     p.CT = (n_head * hd + kNT - 1) / kNT + (n_kv + hpt - 1) / hpt;
     p.big = false;
     p.RT = n_tok == 1 ? (n_seq + kMT - 1) / kMT : n_seq * (n_tok / kBlk + 2);
     const int tiles = p.RT * p.CT;
-    if (kq_tiles(tiles)) {
+    if (kq_tiles(tiles) && !in_place) {
         p.big = true;
         p.RT = (p.RT + 1) / 2;
         p.kps = dim;
@@ -653,7 +654,8 @@ hipError_t launch_qkv_kq(const KvLayerView &L, const int32_t *d_len, const float
     a.n_split = plan.n_split;
     a.n_wg = plan.RT * plan.CT * plan.n_split;
     const int rows = (n_head + 2 * L.H) * L.hd;
-    if (n_tok == 1 && gemv_fits(ggml_type, L.S, dim, rows) && !plan.big) return qkv_gemv(ggml_type, a, part, st);
+    if (n_tok == 1 && !plan.big && !plan.in_place && gemv_fits(ggml_type, L.S, dim, rows))
+        return qkv_gemv(ggml_type, a, part, st);
     const int grid = (a.n_wg + 7) / 8 * 8;
     kq_dispatch(ggml_type, [&](auto tc) {
         constexpr int T = decltype(tc)::value;
@@ -704,7 +706,8 @@ hipError_t launch_qkv(const KvLayerView &L, const int32_t *d_len, const float *x
     a.n_wg = plan.RT * plan.CT * plan.n_split;
     // (the split plans' scratch is at least 256 floats for every K and V column of 32 rows)
     const int form = planes == 2 ? kGemvF16x2 : kGemvF16, rows = (n_head + 2 * L.H) * L.hd;
-    if (n_tok == 1 && gemv_fits(form, L.S, dim, rows) && !plan.big) return qkv_gemv(form, a, part, st);
+    if (n_tok == 1 && !plan.big && !plan.in_place && gemv_fits(form, L.S, dim, rows))
+        return qkv_gemv(form, a, part, st);
     const int grid = (a.n_wg + 7) / 8 * 8;
     if (plan.big) {
         qkv_tile_kernel<0><<<grid, 256, 0, st>>>(a);

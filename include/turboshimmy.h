@@ -175,6 +175,12 @@ int ts_kv_shift(ts_kv *kv, int32_t layer, int32_t seq, int32_t keep_sink, int32_
  * 16-byte aligned, as hipMalloc and torch allocations are; otherwise the call returns
  * TS_ERR_INVALID and launches nothing. */
 
+/* A projection's outputs (q, k, v; act, stash) may share memory with its input where the results
+ * go through partials in the workspace: with f16 rows, under 256 tiles of 32 rows x 256 columns and
+ * a reduction (planes * dim) of 512 or more in whole 256s; with GGUF blocks always, but from 256
+ * tiles on such a call needs a workspace of 32768 bytes a tile (TS_ERR_WORKSPACE with less).  Not in
+ * ts_qkv_append* of a cache whose head_dim is neither 64 nor 128. */
+
 /* RoPE-fused quantize-on-append.  Replaces quantize_kv (sh_quantize_kv.wgsl:39-90, dispatched
  * at layer.rs:1092-1099) plus the RoPE step of attention.rs:196-199.
  * d_k, d_v: [n_seq][n_tok][n_head_kv][head_dim] raw f32.  Token t of sequence s is written
