@@ -201,9 +201,10 @@ struct QkvPlan {
 QkvPlan qkv_plan(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok);
 // GGUF block weights (Q4_K, Q5_K, Q8_0, Q4_0, Q5_0) read in the loop, dim a multiple of 256: the split
 // form with partials in `part` (part_bytes > 0), or with many tiles the tile kernel without any.
-QkvPlan qkv_plan_kq(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok, bool in_place = false);
+QkvPlan qkv_plan_kq(int ggml_type, int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok,
+                    bool in_place = false);
 // The most part_bytes of qkv_plan_kq for 1 to n_tok tokens.
-uint64_t qkv_part_bytes_kq(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok);
+uint64_t qkv_part_bytes_kq(int ggml_type, int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok);
 hipError_t launch_qkv_kq(const KvLayerView &L, const int32_t *d_len, const float *x, int dim, int n_tok,
                          int ggml_type, const void *wq, const void *wk, const void *wv, int n_head,
                          float *q_out, float *k_out, float *v_out, const float *rope, int rope_pairs,
@@ -220,8 +221,9 @@ struct ProjPlan {
     bool in_place = false;  // act or stash shares memory with the input (as QkvPlan)
 };
 ProjPlan proj_plan(int M, int K, int N);
-ProjPlan proj_plan_kq(int M, int K, int N, bool in_place = false);  // block weights, K a multiple of 256
-uint64_t proj_part_bytes_kq(int M, int K, int N);  // the most part_bytes of it for 1 to M rows
+// Block weights, K a multiple of 256; and the most part_bytes of it for 1 to M rows.
+ProjPlan proj_plan_kq(int ggml_type, int M, int K, int N, bool in_place = false);
+uint64_t proj_part_bytes_kq(int ggml_type, int M, int K, int N);
 hipError_t launch_proj_kq(const float *a, int M, int K, int ggml_type, const void *w, int N, float *act,
                           float *stash, const ProjPlan &plan, float *part, hipStream_t st);
 hipError_t launch_proj(const float *a, int M, int K, const uint16_t *w, int N, float *act, float *stash,

@@ -60,8 +60,12 @@ void kq_dispatch(int t, F f) {
 // slices would not split the reduction either, so that the sums keep their bits.  Measured either
 // way on whole blocks of 100 to 600 tokens, 2048 to 4096 wide: below 256 tiles Q4_K, Q5_K and Q4_0
 // lose 0.78-0.99 of their speed (Q8_0 and Q5_0 gain up to 1.2 from 192 on), just above all gain
-// (300 tokens of 4096: 1.01-1.3, 420 of 3072: 1.27-1.57).
-inline bool kq_tiles(int tiles32) { return tiles32 >= 256; }
+// (300 tokens of 4096: 1.01-1.3, 420 of 3072: 1.27-1.57).  At 256 the slices are one full round; Q4_K,
+// the cheapest to decode, keeps them there when they are long (507 rows of 4096 -> 4096: 62.9 us,
+// tiles 65.9; 251 of 8192 -> 8192: 121.7, 129.1; 1019 of 2048 -> 2048: 39.8, 37.2; Q5_K 75.3, 71.8).
+inline bool kq_tiles(int type, int tiles32, int K) {
+    return tiles32 > 256 || (tiles32 == 256 && !(type == kGgmlQ4K && K > 2048));
+}
 
 // Slices of a reduction over K (a multiple of 256) for fewer tiles than that (one slice for more),
 // and the bytes of their partials: splits for about one workgroup per CU (256; 512 and 1024 measured

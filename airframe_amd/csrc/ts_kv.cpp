@@ -703,11 +703,12 @@ struct QkvGenericKq {
     ts::ProjPlan pq, pk;
     uint64_t part_bytes, kv_elems;
 };
-static QkvGenericKq qkv_generic_plan_kq(const ts_kv *kv, int32_t dim, int32_t n_tok, int32_t n_head) {
+static QkvGenericKq qkv_generic_plan_kq(const ts_kv *kv, int32_t ggml_type, int32_t dim, int32_t n_tok,
+                                        int32_t n_head) {
     QkvGenericKq g;
     const int M = kv->d.n_seq * n_tok, hd = kv->d.head_dim;
-    g.pq = ts::proj_plan_kq(M, dim, n_head * hd);
-    g.pk = ts::proj_plan_kq(M, dim, kv->d.n_head_kv * hd);
+    g.pq = ts::proj_plan_kq(ggml_type, M, dim, n_head * hd);
+    g.pk = ts::proj_plan_kq(ggml_type, M, dim, kv->d.n_head_kv * hd);
     g.part_bytes = (std::max(g.pq.part_bytes, g.pk.part_bytes) + 255) / 256 * 256;
     g.kv_elems = (uint64_t)M * kv->d.n_head_kv * hd;
     return g;
@@ -723,11 +724,11 @@ int ts_qkv_gguf_workspace(const ts_kv *kv, int32_t ggml_type, int32_t dim, int32
     // caller sizes its buffer by its longest chunk
     const int S = kv->d.n_seq, hd = kv->d.head_dim, H = kv->d.n_head_kv;
     if (qkv_fused(kv)) {
-        *bytes = ts::qkv_part_bytes_kq(S, H, n_head, hd, dim, n_tok);
+        *bytes = ts::qkv_part_bytes_kq(ggml_type, S, H, n_head, hd, dim, n_tok);
     } else {
-        const uint64_t part = std::max(ts::proj_part_bytes_kq(S * n_tok, dim, n_head * hd),
-                                       ts::proj_part_bytes_kq(S * n_tok, dim, H * hd));
-        *bytes = (part + 255) / 256 * 256 + 2 * qkv_generic_plan_kq(kv, dim, n_tok, n_head).kv_elems * sizeof(float);
+        const uint64_t part = std::max(ts::proj_part_bytes_kq(ggml_type, S * n_tok, dim, n_head * hd),
+                                       ts::proj_part_bytes_kq(ggml_type, S * n_tok, dim, H * hd));
+        *bytes = (part + 255) / 256 * 256 + 2 * qkv_generic_plan_kq(kv, ggml_type, dim, n_tok, n_head).kv_elems * sizeof(float);
     }
     return TS_OK;
 }
@@ -749,7 +750,7 @@ int ts_qkv_append_gguf(ts_kv *kv, int32_t layer, const float *d_x, int32_t dim, 
     if (n_tok == 0) return TS_OK;
     const hipStream_t st = as_stream(stream);
     if (!qkv_fused(kv)) {
-        const QkvGenericKq g = qkv_generic_plan_kq(kv, dim, n_tok, n_head);
+        const QkvGenericKq g = qkv_generic_plan_kq(kv, ggml_type, dim, n_tok, n_head);
         const uint64_t need = g.part_bytes + (d_k ? 0 : 2 * g.kv_elems * sizeof(float));
         if (need > 0 && (!d_workspace || workspace_bytes < need || !aligned16(d_workspace))) return TS_ERR_WORKSPACE;
         float *part = static_cast<float *>(d_workspace);
@@ -767,7 +768,7 @@ int ts_qkv_append_gguf(ts_kv *kv, int32_t layer, const float *d_x, int32_t dim, 
                                          rope->rope_dim / 2, n_tok / 32 + 2, st);
         return hip_status(e);
     }
-    const ts::QkvPlan plan = ts::qkv_plan_kq(kv->d.n_seq, kv->d.n_head_kv, n_head, kv->d.head_dim, dim, n_tok,
+    const ts::QkvPlan plan = ts::qkv_plan_kq(ggml_type, kv->d.n_seq, kv->d.n_head_kv, n_head, kv->d.head_dim, dim, n_tok,
                                              qkv_in_place(kv, d_x, dim, n_tok, n_head, d_q, d_k, d_v));
     if (plan.part_bytes > 0 && (!d_workspace || workspace_bytes < plan.part_bytes || !aligned16(d_workspace)))
         return TS_ERR_WORKSPACE;
@@ -786,7 +787,7 @@ static bool proj_in_place(const float *d_attn, int32_t n_tok, int32_t attn_dim, 
 int ts_attn_out_proj_gguf_workspace(int32_t ggml_type, int32_t n_tok, int32_t attn_dim, int32_t dim, uint64_t *bytes) {
     if (!bytes || n_tok < 0 || attn_dim <= 0 || attn_dim % 256 != 0 || dim <= 0) return TS_ERR_INVALID;
     if (!kq_type_ok(ggml_type)) return TS_ERR_UNSUPPORTED;
-    *bytes = n_tok > 0 ? ts::proj_part_bytes_kq(n_tok, attn_dim, dim) : 0;  // (any rows up to n_tok)
+    *bytes = n_tok > 0 ? ts::proj_part_bytes_kq(ggml_type, n_tok, attn_dim, dim) : 0;  // (any rows up to n_tok)
     return TS_OK;
 }
 
@@ -799,7 +800,7 @@ int ts_attn_out_proj_gguf(const float *d_attn, int32_t n_tok, int32_t attn_dim, 
     if (!kq_type_ok(ggml_type)) return TS_ERR_UNSUPPORTED;
     if (n_tok == 0) return TS_OK;
     const ts::ProjPlan plan =
-        ts::proj_plan_kq(n_tok, attn_dim, dim, proj_in_place(d_attn, n_tok, attn_dim, dim, d_act, d_stash));
+        ts::proj_plan_kq(ggml_type, n_tok, attn_dim, dim, proj_in_place(d_attn, n_tok, attn_dim, dim, d_act, d_stash));
     if (plan.part_bytes > 0 && (!d_workspace || workspace_bytes < plan.part_bytes || !aligned16(d_workspace)))
         return TS_ERR_WORKSPACE;
     return hip_status(ts::launch_proj_kq(d_attn, n_tok, attn_dim, ggml_type, d_wo, dim, d_act, d_stash, plan,

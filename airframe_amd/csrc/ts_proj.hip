@@ -257,13 +257,13 @@ ProjPlan proj_plan(int M, int K, int N) {
     return p;
 }
 
-ProjPlan proj_plan_kq(int M, int K, int N, bool in_place) {
+ProjPlan proj_plan_kq(int ggml_type, int M, int K, int N, bool in_place) {
     ProjPlan p;
     p.in_place = in_place;
     p.CT = (N + kPT - 1) / kPT;
     p.RT = (M + 31) / 32;
     const int tiles = p.RT * p.CT;
-    if (kq_tiles(tiles) && !in_place) {
+    if (kq_tiles(ggml_type, tiles, K) && !in_place) {
         p.RT = (M + 63) / 64;
         p.kps = K;
         p.n_split = 1;
@@ -277,10 +277,11 @@ ProjPlan proj_plan_kq(int M, int K, int N, bool in_place) {
     return p;
 }
 
-uint64_t proj_part_bytes_kq(int M, int K, int N) {
+uint64_t proj_part_bytes_kq(int ggml_type, int M, int K, int N) {
     const int CT = (N + kPT - 1) / kPT, RT = (M + 31) / 32;
     uint64_t most = 0;
-    for (int rt = 1; rt <= RT && !kq_tiles(rt * CT); rt++) most = std::max(most, kq_slices(rt * CT, K).bytes);
+    for (int rt = 1; rt <= RT && !kq_tiles(ggml_type, rt * CT, K); rt++)
+        most = std::max(most, kq_slices(rt * CT, K).bytes);
     return most;
 }
 

@@ -586,7 +586,7 @@ QkvPlan qkv_plan(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok) {
     return p;
 }
 
-QkvPlan qkv_plan_kq(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok, bool in_place) {
+QkvPlan qkv_plan_kq(int ggml_type, int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok, bool in_place) {
     QkvPlan p;
     p.in_place = in_place;
     const int hpt = 128 / hd;
@@ -594,7 +594,7 @@ QkvPlan qkv_plan_kq(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok,
     p.big = false;
     p.RT = n_tok == 1 ? (n_seq + kMT - 1) / kMT : n_seq * (n_tok / kBlk + 2);
     const int tiles = p.RT * p.CT;
-    if (kq_tiles(tiles) && !in_place) {
+    if (kq_tiles(ggml_type, tiles, dim) && !in_place) {
         p.big = true;
         p.RT = (p.RT + 1) / 2;
         p.kps = dim;
@@ -609,11 +609,11 @@ QkvPlan qkv_plan_kq(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok,
     return p;
 }
 
-uint64_t qkv_part_bytes_kq(int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok) {
+uint64_t qkv_part_bytes_kq(int ggml_type, int n_seq, int n_kv, int n_head, int hd, int dim, int n_tok) {
     uint64_t most = 0;
     // (a token count sets the tiles through n_tok / kBlk alone, apart from one token's)
     for (int t = 1; t <= n_tok; t = t == 1 ? 2 : t < kBlk ? kBlk : t + kBlk) {
-        const QkvPlan p = qkv_plan_kq(n_seq, n_kv, n_head, hd, dim, t);
+        const QkvPlan p = qkv_plan_kq(ggml_type, n_seq, n_kv, n_head, hd, dim, t);
         if (t > 1 && p.big) break;
         most = std::max(most, p.part_bytes);
     }
