@@ -1493,7 +1493,7 @@ DecodePlan decode_plan_even(const int32_t *n_ctx, int n_seq, int n_kv, int G, in
         p.g4 = p.chunk >= 1024;
     }
     if (!p.g4) p.chunk = even_chunk(n_ctx, n_seq, n_kv * ((G + 7) / 8), 2 * n_cu);
-    p.n_split = (max_ctx + p.chunk - 1) / p.chunk;
+    p.n_split = p.even_split = (max_ctx + p.chunk - 1) / p.chunk;
     return p;
 }
 
@@ -1530,7 +1530,7 @@ DecodePlan decode_plan(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_c
         p.g4 = false;
         p.nw = n_win <= 8 ? 8 : 16;
         p.chunk = (max_ctx + 63) / 64 * 64;
-        p.n_split = 1;
+        p.n_split = p.even_split = 1;
         return p;
     }
     const float bytes_us = (float)total * n_kv * (stored_hd + 8) / kDecodeBytesUs;
@@ -1549,6 +1549,7 @@ DecodePlan decode_plan(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_c
     };
     const DecodePlan even = decode_plan_even(n_ctx, n_seq, n_kv, G, n_cu, stored_hd);
     weigh(even.chunk, even.g4);
+    p.even_split = even.n_split;
     const int most = std::min((max_ctx + kMinChunk - 1) / kMinChunk, decode_cap(n_kv, max_ctx, n_cu));
     for (int k = 1; k <= most; k = k == most ? k + 1 : std::min(most, k + (k < 8 ? 1 : k / 4))) {
         // (a few positions to spare, so that the plan of a length that is a multiple of k windows

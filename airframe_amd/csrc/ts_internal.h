@@ -160,13 +160,15 @@ struct DecodePlan {
     int n_split;  // splits of the longest sequence (grid.x)
     bool g4;      // the integer kernel, G <= 16 (QK^T on v_mfma_i32_16x16x64_i8)
     int nw;       // waves per workgroup of the 16x16 kernel (4, or 8 / 16 without a split)
+    int even_split;  // splits of the plan that spreads the context evenly (decode_plan_even, or 1 for
+                     // a wide workgroup per stream): whether a caller has to give a workspace
 };
 // n_ctx: keys per sequence (len + 1), on the host; n_cu: compute units of the device;
 // stored_hd: the stored head dim (64, 128 or 256); fused: the launch appends the new token
 // (its position is scored from registers, not streamed).
 DecodePlan decode_plan(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_cu, int stored_hd, bool fused);
-// The plan that ts_attn_decode_append_noalloc falls back to when the partials of decode_plan's do
-// not fit its scratch array: fewer splits for some batches.
+// The plan to fall back to when the partials of decode_plan's do not fit what there is (the library's
+// scratch array, or no workspace from a caller who needs none): fewer splits for some batches.
 DecodePlan decode_plan_even(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_cu, int stored_hd);
 // The integer kernel takes up to 16 query heads per kv head on stored rows up to 128 dims, 8 on
 // 256-dim rows.

@@ -475,16 +475,18 @@ static int attn_decode(const ts_kv *kv, int32_t layer, const float *d_q, int32_t
                                           kv->n_cu, kv->hdp, k_new != nullptr);
     // partials [S][n_head][n_split][hd], then m and l [S][n_head][n_split]
     const uint64_t per_split = (uint64_t)kv->d.n_seq * n_head * (kv->hdp + 2) * sizeof(float);
-    if (noalloc && plan.n_split > 1 && plan.n_split * per_split > workspace_bytes)
+    uint64_t need = plan.n_split * per_split;
+    // a caller's: plan.n_split <= decode_cap(max_seq), the count the workspace was sized for
+    if (!noalloc) ts_attn_decode_workspace(kv, n_head, &need);
+    const int rc_ws = !d_workspace || workspace_bytes < need ? TS_ERR_WORKSPACE
+                      : !aligned16(d_workspace)              ? TS_ERR_INVALID
+                                                             : TS_OK;
+    // Which calls of a caller have to bring a workspace does not change with the plan that is taken
+    // in the end.
+    if (!noalloc && plan.even_split > 1 && rc_ws != TS_OK) return rc_ws;
+    if (plan.n_split > 1 && rc_ws != TS_OK) {
         plan = ts::decode_plan_even(ctx.data(), kv->d.n_seq, kv->d.n_head_kv, n_head / kv->d.n_head_kv, kv->n_cu, kv->hdp);
-    if (plan.n_split > 1) {
-        uint64_t need = 0;
-        if (noalloc)
-            need = plan.n_split * per_split;
-        else  // plan.n_split <= decode_cap(max_seq), the count the workspace was sized for
-            ts_attn_decode_workspace(kv, n_head, &need);
-        if (!d_workspace || workspace_bytes < need) return TS_ERR_WORKSPACE;
-        if (!aligned16(d_workspace)) return TS_ERR_INVALID;
+        if (plan.n_split > 1 && (!noalloc || plan.n_split * per_split > workspace_bytes)) return rc_ws;
     }
     // An eager call takes the host's lengths as launch arguments (the device's agree with them
     // unless a captured call changed them); one being captured reads the device lengths, so
