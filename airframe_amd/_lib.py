@@ -60,6 +60,7 @@ SIGNATURES = {
     "ts_append_quant": (ctypes.c_int, [_vp, _i32, _vp, _vp, _i32, _vp, _vp]),
     "ts_requant_all": (ctypes.c_int, [_vp, _i32, _vp, _vp, _i32, _i32, _vp, _vp]),
     "ts_attn_decode_workspace": (ctypes.c_int, [_vp, _i32, _u64p]),
+    "ts_attn_decode_plan": (ctypes.c_int, [_i32p, _i32, _i32, _i32, _i32, _i32, _i32, _i32p]),
     "ts_attn_decode": (ctypes.c_int, [_vp, _i32, _vp, _i32, _vp, _f, _vp, _vp, ctypes.c_uint64, _vp]),
     "ts_attn_decode_append": (ctypes.c_int, [_vp, _i32, _vp, _vp, _vp, _i32, _vp, _f, _vp, _vp,
                                              ctypes.c_uint64, _vp]),

@@ -454,6 +454,20 @@ int ts_attn_decode_workspace(const ts_kv *kv, int32_t n_head, uint64_t *bytes) {
     return TS_OK;
 }
 
+int ts_attn_decode_plan(const int32_t *n_ctx, int32_t n_seq, int32_t n_head_kv, int32_t n_head, int32_t head_dim,
+                        int32_t n_cu, int32_t fused, int32_t *plan) {
+    if (!n_ctx || !plan || n_seq <= 0 || n_head_kv <= 0 || n_head <= 0 || n_head % n_head_kv != 0 || head_dim <= 0 ||
+        head_dim > 256 || head_dim % 8 != 0 || n_cu <= 0 || *std::min_element(n_ctx, n_ctx + n_seq) < 1)
+        return TS_ERR_INVALID;
+    const ts::DecodePlan p =
+        ts::decode_plan(n_ctx, n_seq, n_head_kv, n_head / n_head_kv, n_cu, stored_head_dim(head_dim), fused != 0);
+    plan[0] = p.g4;
+    plan[1] = p.nw;
+    plan[2] = p.chunk;
+    plan[3] = p.n_split;
+    return TS_OK;
+}
+
 // Shared by ts_attn_decode, ts_attn_decode_append and ts_attn_decode_append_noalloc
 // (k_new/v_new null for the first).  d_workspace: the caller's workspace of workspace_bytes,
 // checked against the worst case the workspace query promises; or, with noalloc, the

@@ -31,6 +31,14 @@ def _ptr(t: torch.Tensor, dtype: torch.dtype, what: str) -> ctypes.c_void_p:
     return ctypes.c_void_p(t.data_ptr())
 
 
+def decode_plan(n_ctx, n_head_kv: int, n_head: int, head_dim: int, n_cu: int, fused: bool = True) -> dict:
+    """How a decode call over n_ctx keys per sequence (lengths + 1) divides its work (ts_attn_decode_plan)."""
+    ctx, plan = (ctypes.c_int32 * len(n_ctx))(*n_ctx), (ctypes.c_int32 * 4)()
+    check("ts_attn_decode_plan",
+          load().ts_attn_decode_plan(ctx, len(n_ctx), n_head_kv, n_head, head_dim, n_cu, fused, plan))
+    return {"integer": bool(plan[0]), "waves": plan[1], "chunk": plan[2], "splits": plan[3]}
+
+
 class RopeTable:
     """PreflightResources' RoPE table (preflight.rs:71-142): host-computed cos/sin, uploaded."""
 

@@ -908,61 +908,17 @@ def run_stream_ceiling(args, cfg):
     return res
 
 
-def _split_kernel_name(cfg, n_cu=256):
-    """Which split kernel the library launches for this shape: decode_plan and the dispatch
-    rule of launch_decode (ts_decode.hip), restated for the bench label (the step's starting
-    lengths; MI355X has 256 CUs)."""
+def _split_kernel_name(cfg, fused, n_cu=256):
+    """Which split kernel the library launches for this shape at the step's starting lengths
+    (MI355X has 256 CUs)."""
+    from airframe_amd.kv_cache import decode_plan
     if "ragged" in cfg:
         rng = np.random.default_rng(2024)
         ctx = [int(x) + 1 for x in rng.integers(cfg["ragged"][0], cfg["ragged"][1], size=cfg["batch"])]
     else:
         ctx = [cfg["ctx"] + 1] * cfg["batch"]
-
-    hd, n_kv, G = cfg["hd"], cfg["n_kv"], cfg["n_head"] // cfg["n_kv"]
-    stored = 64 if hd <= 64 else 128 if hd <= 128 else 256
-    top, total, S = max(ctx), sum(ctx), len(ctx)
-    n_win, wmax = -(-(top - 1) // 64), {64: 16, 128: 8, 256: 4}[stored]
-    if 4 < n_win <= wmax and S * n_kv * -(-G // 8) <= n_cu:
-        return "decode_split_kernel"
-    halves = -(-G // 4)
-    heads = 1.0 if halves <= 1 else 1.5 if halves == 2 else 2.5
-    cost = {  # fixed, per round, positions per round, workgroups at once, streams
-        1: ((5.0 if halves <= 1 else 7.5 if halves == 2 else 13.0) + (2.5 if stored == 256 else 0.0), (1.4 if halves <= 1 else 1.8 if halves == 2 else 3.2) if stored == 64
-            else (1.75 if stored == 256 else 0.95) * heads, 512 if stored == 64 else 256, n_cu, n_kv),
-        0: (4.0, {64: 1.33, 128: 1.55, 256: 3.2}[stored] * (1.4 if G > 4 else 1.0), 256, 1.25 * n_cu,
-            n_kv * -(-G // 8)),
-    }
-    bytes_us = total * n_kv * (stored + 8) / 6.5e6
-    most = min(-(-top // 256), min(-(-top // 64), 2 * n_cu // n_kv + 2))
-
-    def even(target, streams):
-        busy = lambda c: sum(-(-x // c) for x in ctx) * streams
-        hi = max(256, -(-top // 64) * 64)
-        lo = -(-min(hi, max(256, -(-total * streams // target))) // 64) * 64
-        c = lo
-        while c < hi and busy(c) > target:
-            c += 64
-        return lo if busy(c) > target else c  # no chunk meets the target: the balanced one
-
-    kinds = (1, 0) if G <= (16 if stored <= 128 else 8) else (0,)  # decode_int_gmax (ts_internal.h)
-    c4 = even(n_cu - n_cu // 8, n_kv)
-    tries, k = [(c4, 1) if kinds[0] and c4 >= 1024 else (even(2 * n_cu, cost[0][4]), 0)], 1
-    while k <= most:
-        tries += [(-(-(-(-top // k) + (4 if k > 1 else 0)) // 64) * 64, kind) for kind in kinds]
-        k = k + 1 if k == most else min(most, k + (1 if k < 8 else k // 4))
-    best, g4 = None, 0
-    for chunk, kind in tries:
-        fixed, rnd, span, at_once, streams = cost[kind]
-        splits = [-(-x // chunk) for x in ctx]
-        cus = 0.875 if min(splits) != max(splits) else 1.0
-        us = longest = fixed + rnd * -(-min(chunk, top) // span)
-        if sum(splits) * streams > cus * n_cu:
-            work = sum(splits) * streams * (fixed + 0.5 * rnd) + rnd * total * streams / span
-            us = max(us, work / (cus * at_once) + 0.5 * longest)
-        us = max(us, bytes_us + fixed) + (3.5 if max(splits) > 1 else 0.0)
-        if best is None or us < 0.98 * best:
-            best, g4 = us, kind
-    return "decode_split4_kernel" if g4 else "decode_split_kernel"
+    plan = decode_plan(ctx, cfg["n_kv"], cfg["n_head"], cfg["hd"], n_cu, fused)
+    return "decode_split4_kernel" if plan["integer"] else "decode_split_kernel"
 
 
 def main():
@@ -1200,7 +1156,7 @@ def main():
     gbs = r["step_bytes"] / (r["ms_step"] * 1e-3) / 1e9
     tok_s = B / (r["ms_step"] * 1e-3)
     ach = r["kernel_bytes"] / (r["kernel_ms"] * 1e-3) / 1e9
-    split_name = _split_kernel_name(cfg)
+    split_name = _split_kernel_name(cfg, not args.separate)
     roof = {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(ach / HBM_PEAK_GBS, 4), "traffic": traffic,
             "traffic_source": (f"profiles/decode_cfg{args.config}.md (rocprofv3 --pmc FETCH_SIZE / "

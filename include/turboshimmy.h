@@ -201,6 +201,14 @@ int ts_requant_all(ts_kv *kv, int32_t layer, const float *d_k_cache, const float
  * to max_seq).  Host only. */
 int ts_attn_decode_workspace(const ts_kv *kv, int32_t n_head, uint64_t *bytes);
 
+/* How a decode call divides its work: n_ctx[s] keys of sequence s (its length + 1), on a device of n_cu
+ * compute units; fused: the call appends the new token (ts_attn_decode_append*).  plan[0]: 1 for the
+ * kernel whose QK^T runs on integers, 0 for the other; plan[1]: waves of the other's workgroups;
+ * plan[2]: positions per split; plan[3]: splits of the longest sequence (more than one: a combine
+ * launch follows).  For labels and tests; host only. */
+int ts_attn_decode_plan(const int32_t *n_ctx, int32_t n_seq, int32_t n_head_kv, int32_t n_head, int32_t head_dim,
+                        int32_t n_cu, int32_t fused, int32_t *plan);
+
 /* INT4 GQA decode attention.  Replaces main_attn_out_int4 (sh_layer_v1_int4.wgsl:1042-1143,
  * dispatched at layer.rs:1100-1107) with the CPU path's semantics (attention.rs:236-313).
  * d_q: [n_seq][n_head][head_dim] raw f32 for the token just appended; it is rotated at

@@ -1,0 +1,47 @@
+"""The plan of a decode call (kernel, positions per split, splits) through the library's host-only query:
+which shapes the weighed plan changes, and to what."""
+import ctypes
+
+import pytest
+
+import airframe_amd
+from airframe_amd import _lib
+from airframe_amd.kv_cache import decode_plan
+
+N_CU = 256
+
+
+def lens(n_seq, lo, hi):
+    """Keys of n_seq sequences spread evenly from lo to hi."""
+    return [lo + (hi - lo) * s // max(1, n_seq - 1) for s in range(n_seq)]
+
+
+def plan(n_seq, n_kv, G, hd, lo, hi):
+    p = decode_plan(lens(n_seq, lo, hi), n_kv, n_kv * G, hd, N_CU)
+    return ("integer" if p["integer"] else "16x16", p["waves"], p["chunk"], p["splits"])
+
+
+@pytest.mark.parametrize("shape,want", [
+    ((1, 8, 4, 64, 513, 513), ("16x16", 8, 576, 1)),         # a wide workgroup per stream
+    ((1, 8, 3, 128, 4172, 4172), ("16x16", 4, 256, 17)),     # short splits, two workgroups a CU
+    ((32, 8, 4, 128, 8193, 8193), ("integer", 4, 8256, 1)),  # a workgroup per stream and CU
+    ((32, 8, 4, 128, 701, 1532), ("integer", 4, 1536, 1)),   # ragged, about as many streams as CUs: no split
+    ((32, 8, 4, 64, 1000, 3000), ("integer", 4, 3008, 1)),
+    ((8, 8, 2, 256, 1000, 4000), ("integer", 4, 1024, 4)),
+    ((2, 8, 4, 128, 6369, 6369), ("integer", 4, 448, 15)),   # integer splits of less than four rounds
+    ((60, 2, 40, 128, 90, 90), ("16x16", 4, 256, 1)),        # more query heads than the integer kernel takes
+])
+def test_plan(shape, want):
+    assert plan(*shape) == want
+
+
+def test_query_refuses_bad_arguments():
+    L = airframe_amd.load()
+    i32 = ctypes.c_int32
+    ctx, out = (i32 * 2)(5, 9), (i32 * 4)()
+    assert L.ts_attn_decode_plan(ctx, 2, 8, 32, 128, N_CU, 1, out) == _lib.TS_OK
+    for bad in ((None, 2, 8, 32, 128, N_CU, 1, out), (ctx, 0, 8, 32, 128, N_CU, 1, out), (ctx, 2, 0, 32, 128, N_CU, 1, out),
+                (ctx, 2, 8, 31, 128, N_CU, 1, out), (ctx, 2, 8, 32, 260, N_CU, 1, out), (ctx, 2, 8, 32, 60, N_CU, 1, out),
+                (ctx, 2, 8, 32, 128, 0, 1, out), (ctx, 2, 8, 32, 128, N_CU, 1, None),
+                ((i32 * 2)(0, 9), 2, 8, 32, 128, N_CU, 1, out)):
+        assert L.ts_attn_decode_plan(*bad) == _lib.TS_ERR_INVALID
