@@ -1524,9 +1524,12 @@ DecodePlan decode_plan(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_c
     // positions + the new token), 16 waves 10.1, four-wave splits and a combine 10.5.  More than
     // one window per wave does not pay: 8.5 windows per wave took 26.6 us per layer on config 2's
     // shape against 10.0 with splits and a combine.
+    // (Not in the place of the integer kernel without a split, which serves about as many streams as
+    // CUs: 256 streams of 1000 64-dim positions 9.8 us a layer, 12.6 with 16 waves.)
+    const DecodePlan even = decode_plan_even(n_ctx, n_seq, n_kv, G, n_cu, stored_hd);
     const int n_win = (max_ctx - (fused ? 1 : 0) + 63) / 64;
     const int wmax = stored_hd <= 64 ? 16 : stored_hd <= 128 ? 8 : 4;
-    if (n_win > 4 && n_win <= wmax && (int64_t)n_seq * n_kv * groups <= n_cu) {
+    if (!even.g4 && n_win > 4 && n_win <= wmax && (int64_t)n_seq * n_kv * groups <= n_cu) {
         p.g4 = false;
         p.nw = n_win <= 8 ? 8 : 16;
         p.chunk = (max_ctx + 63) / 64 * 64;
@@ -1547,7 +1550,6 @@ DecodePlan decode_plan(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_c
             p.chunk = chunk;
         }
     };
-    const DecodePlan even = decode_plan_even(n_ctx, n_seq, n_kv, G, n_cu, stored_hd);
     weigh(even.chunk, even.g4);
     p.even_split = even.n_split;
     const int most = std::min((max_ctx + kMinChunk - 1) / kMinChunk, decode_cap(n_kv, max_ctx, n_cu));

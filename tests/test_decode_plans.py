@@ -35,6 +35,14 @@ def test_plan(shape, want):
     assert plan(*shape) == want
 
 
+@pytest.mark.parametrize("n_seq,n_kv,G", [(32, 8, 1), (17, 8, 4), (28, 8, 8), (8, 32, 1), (64, 4, 4), (26, 8, 8)])
+@pytest.mark.parametrize("ctx", [961, 1000, 1024])
+def test_integer_kernel_keeps_unsplit_streams(n_seq, n_kv, G, ctx):
+    """About as many streams as CUs of one round of the integer kernel: the wide workgroups of the 16x16
+    kernel take a third longer there."""
+    assert plan(n_seq, n_kv, G, 64, ctx, ctx) == ("integer", 4, 1024, 1)
+
+
 def test_query_refuses_bad_arguments():
     L = airframe_amd.load()
     i32 = ctypes.c_int32
