@@ -1397,21 +1397,29 @@ windows_done:
 namespace {
 constexpr int kMinChunk = 256;  // splits shorter than this leave waves without a window
 
+// Splits of `chunk` positions of all sequences; *idle: some sequence has fewer than the longest, whose
+// grid then holds workgroups without work.
+int64_t count_splits(const int32_t *n_ctx, int n_seq, int max_ctx, int chunk, bool *idle) {
+    *idle = false;
+    if (chunk >= max_ctx) return n_seq;
+    const float inv = 1.0f / chunk;
+    const int most = (max_ctx + chunk - 1) / chunk;
+    int n = 0, fewer = 0;  // (32 bits and no branch: the loop runs on vectors)
+    for (int s = 0; s < n_seq; s++) {
+        const int c = (int)((n_ctx[s] - 0.5f) * inv) + 1;
+        n += c;
+        fewer |= c ^ most;
+    }
+    *idle = fewer != 0;
+    return n;
+}
+
 // The chunk that spreads a batch's context evenly: the smallest multiple of 64 for which the busy
 // workgroups of the whole batch, n_kv * sum_s ceil(n_ctx[s] / chunk), fit in `target`; with
 // more streams than the target, the batch's work over the target.
-int even_chunk(const int32_t *n_ctx, int n_seq, int n_kv, int target) {
-    int64_t total = 0;
-    int max_ctx = 1;
-    for (int s = 0; s < n_seq; s++) {
-        total += n_ctx[s];
-        max_ctx = std::max(max_ctx, (int)n_ctx[s]);
-    }
-    auto busy = [&](int chunk) {
-        int64_t n = 0;
-        for (int s = 0; s < n_seq; s++) n += (n_ctx[s] + chunk - 1) / chunk;
-        return n * n_kv;
-    };
+int even_chunk(const int32_t *n_ctx, int n_seq, int n_kv, int target, int64_t total, int max_ctx) {
+    bool idle;
+    auto busy = [&](int chunk) { return count_splits(n_ctx, n_seq, max_ctx, chunk, &idle) * n_kv; };
     const int hi_c = std::max(kMinChunk, (max_ctx + 63) / 64 * 64);
     int lo_c = (int)std::min<int64_t>(hi_c, std::max<int64_t>(kMinChunk, (total * n_kv + target - 1) / target));
     lo_c = (lo_c + 63) / 64 * 64;
@@ -1460,20 +1468,14 @@ constexpr float kDecodeBytesUs = 6.5e6f;  // bytes a us that all CUs stream toge
 // dispatcher does not place a workgroup on just any free CU of its XCD.
 float plan_us(const DecodeCost &k, const int32_t *n_ctx, int n_seq, int streams, int64_t total, int max_ctx, int chunk,
               int n_cu, float bytes_us) {
-    const float inv = 1.0f / chunk;
     const int most = (max_ctx + chunk - 1) / chunk;
-    int64_t n = 0;
-    bool idle = false;
-    for (int s = 0; s < n_seq; s++) {
-        const int c = (int)((n_ctx[s] - 0.5f) * inv) + 1;
-        n += c;
-        idle |= c != most;
-    }
+    bool idle;
+    const int64_t busy = count_splits(n_ctx, n_seq, max_ctx, chunk, &idle) * streams;
     const float cus = idle ? 0.875f : 1.0f;
     const float longest = k.fixed + k.round * ((std::min(chunk, max_ctx) + k.span - 1) / k.span);
     float us = longest;
-    if (n * streams > cus * n_cu) {
-        const float work = n * streams * (k.fixed + 0.5f * k.round) + k.round * total * streams / k.span;
+    if (busy > cus * n_cu) {
+        const float work = busy * (k.fixed + 0.5f * k.round) + k.round * total * streams / k.span;
         us = std::max(us, work / (cus * k.at_once) + 0.5f * longest);
     }
     return std::max(us, bytes_us + k.fixed) + (most > 1 ? kCombineUs : 0.0f);
@@ -1482,19 +1484,34 @@ float plan_us(const DecodeCost &k, const int32_t *n_ctx, int n_seq, int streams,
 
 // The batch's context spread evenly (even_chunk) over 7/8 of the CUs for the integer kernel, or, when
 // its splits would be short, over twice the CUs for the 16x16 kernel.
-DecodePlan decode_plan_even(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_cu, int stored_hd) {
+static DecodePlan even_plan(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_cu, int stored_hd, int64_t total,
+                            int max_ctx) {
     DecodePlan p;
     p.nw = 4;
     p.g4 = false;
-    int max_ctx = 1;
-    for (int s = 0; s < n_seq; s++) max_ctx = std::max(max_ctx, (int)n_ctx[s]);
     if (G <= decode_int_gmax(stored_hd)) {
-        p.chunk = even_chunk(n_ctx, n_seq, n_kv, n_cu - n_cu / 8);
+        p.chunk = even_chunk(n_ctx, n_seq, n_kv, n_cu - n_cu / 8, total, max_ctx);
         p.g4 = p.chunk >= 1024;
     }
-    if (!p.g4) p.chunk = even_chunk(n_ctx, n_seq, n_kv * ((G + 7) / 8), 2 * n_cu);
+    if (!p.g4) p.chunk = even_chunk(n_ctx, n_seq, n_kv * ((G + 7) / 8), 2 * n_cu, total, max_ctx);
     p.n_split = p.even_split = (max_ctx + p.chunk - 1) / p.chunk;
     return p;
+}
+
+static void context_of(const int32_t *n_ctx, int n_seq, int64_t &total, int &max_ctx) {
+    total = 0;
+    max_ctx = 1;
+    for (int s = 0; s < n_seq; s++) {
+        max_ctx = std::max(max_ctx, (int)n_ctx[s]);
+        total += n_ctx[s];
+    }
+}
+
+DecodePlan decode_plan_even(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_cu, int stored_hd) {
+    int64_t total;
+    int max_ctx;
+    context_of(n_ctx, n_seq, total, max_ctx);
+    return even_plan(n_ctx, n_seq, n_kv, G, n_cu, stored_hd, total, max_ctx);
 }
 
 // Split plan: the kernel and the split length whose estimate is the lowest, among the batch's
@@ -1507,12 +1524,9 @@ DecodePlan decode_plan_even(const int32_t *n_ctx, int n_seq, int n_kv, int G, in
 // with 256-dim rows 36.2 us on the 16x16 kernel, 19.3 in integer splits of 832; one sequence of
 // 20000 with 24 query heads 17.2 us a layer, 12.4.)
 DecodePlan decode_plan(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_cu, int stored_hd, bool fused) {
-    int max_ctx = 1;
-    int64_t total = 0;
-    for (int s = 0; s < n_seq; s++) {
-        max_ctx = std::max(max_ctx, (int)n_ctx[s]);
-        total += n_ctx[s];
-    }
+    int max_ctx;
+    int64_t total;
+    context_of(n_ctx, n_seq, total, max_ctx);
     DecodePlan p;
     p.nw = 4;
     const int groups = (G + 7) / 8;  // head groups of the 16x16 kernel
@@ -1526,7 +1540,7 @@ DecodePlan decode_plan(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_c
     // shape against 10.0 with splits and a combine.
     // (Not in the place of the integer kernel without a split, which serves about as many streams as
     // CUs: 256 streams of 1000 64-dim positions 9.8 us a layer, 12.6 with 16 waves.)
-    const DecodePlan even = decode_plan_even(n_ctx, n_seq, n_kv, G, n_cu, stored_hd);
+    const DecodePlan even = even_plan(n_ctx, n_seq, n_kv, G, n_cu, stored_hd, total, max_ctx);
     const int n_win = (max_ctx - (fused ? 1 : 0) + 63) / 64;
     const int wmax = stored_hd <= 64 ? 16 : stored_hd <= 128 ? 8 : 4;
     if (!even.g4 && n_win > 4 && n_win <= wmax && (int64_t)n_seq * n_kv * groups <= n_cu) {
@@ -1539,19 +1553,21 @@ DecodePlan decode_plan(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_c
     const float bytes_us = (float)total * n_kv * (stored_hd + 8) / kDecodeBytesUs;
     const bool integer = G <= decode_int_gmax(stored_hd);
     const DecodeCost ki = int_cost(G, stored_hd, n_cu), kf = f16_cost(G, stored_hd, n_cu);
-    float best = 0.0f;
-    p.chunk = 0;
+    auto time = [&](int chunk, bool g4) {
+        return plan_us(g4 ? ki : kf, n_ctx, n_seq, n_kv * (g4 ? 1 : groups), total, max_ctx, chunk, n_cu, bytes_us);
+    };
+    p = even;
+    float best = time(even.chunk, even.g4);
     auto weigh = [&](int chunk, bool g4) {
-        const float us = g4 ? plan_us(ki, n_ctx, n_seq, n_kv, total, max_ctx, chunk, n_cu, bytes_us)
-                            : plan_us(kf, n_ctx, n_seq, n_kv * groups, total, max_ctx, chunk, n_cu, bytes_us);
-        if (p.chunk == 0 || us < 0.98f * best) {
-            best = us;
+        const float t = time(chunk, g4);
+        if (t < 0.98f * best) {
+            best = t;
             p.g4 = g4;
             p.chunk = chunk;
         }
     };
-    weigh(even.chunk, even.g4);
-    p.even_split = even.n_split;
+    // (no plan is estimated below the bytes and either kernel's fixed part)
+    if (0.98f * best <= bytes_us + std::min(ki.fixed, kf.fixed)) return p;
     const int most = std::min((max_ctx + kMinChunk - 1) / kMinChunk, decode_cap(n_kv, max_ctx, n_cu));
     for (int k = 1; k <= most; k = k == most ? k + 1 : std::min(most, k + (k < 8 ? 1 : k / 4))) {
         // (a few positions to spare, so that the plan of a length that is a multiple of k windows
