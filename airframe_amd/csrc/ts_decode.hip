@@ -1574,7 +1574,9 @@ DecodePlan decode_plan(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_c
         // outlives the next tokens, as a captured one has to)
         const int chunk = ((max_ctx + k - 1) / k + (k > 1 ? 4 : 0) + 63) / 64 * 64;
         if (integer) weigh(chunk, true);
-        weigh(chunk, false);
+        // (The 16x16 kernel never in the place of an even plan on the integer one: without splits a tenth
+        // more error against 64 bits, 3.3e-7 and 3.7e-7 over 28 to 75 sequences of 700 to 3000.)
+        if (!even.g4) weigh(chunk, false);
     }
     p.n_split = (max_ctx + p.chunk - 1) / p.chunk;
     return p;

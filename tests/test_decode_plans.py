@@ -44,6 +44,14 @@ def test_integer_kernel_keeps_unsplit_streams(n_seq, n_kv, G, ctx):
     assert plan(n_seq, n_kv, G, 64, ctx, ctx) == ("integer", 4, 1024, 1)
 
 
+@pytest.mark.parametrize("shape", [(52, 8, 8, 128, 722, 1444), (43, 8, 5, 128, 1322, 1322), (20, 2, 16, 128, 4836, 4836),
+                                   (2, 32, 1, 128, 2964, 2964), (14, 1, 8, 128, 15698, 15698)])
+def test_integer_kernel_is_not_replaced(shape):
+    """The integer kernel's scores are exact before one rounding: where the evenly spread context is its, the 16x16
+    kernel (a tenth more error) does not take over."""
+    assert plan(*shape)[0] == "integer"
+
+
 def test_planning_a_large_batch_of_short_sequences_is_cheap():
     """The host sets the pace of such calls, and every layer of a step plans again."""
     L = airframe_amd.load()
