@@ -1466,19 +1466,52 @@ constexpr float kDecodeBytesUs = 6.5e6f;  // bytes a us that all CUs stream toge
 // the bytes.  Only 7/8 of the CUs count when the grid holds idle workgroups (splits past a
 // shorter sequence's end): busy ones then wait 9-20 us for a CU that others leave, since the
 // dispatcher does not place a workgroup on just any free CU of its XCD.
-float plan_us(const DecodeCost &k, const int32_t *n_ctx, int n_seq, int streams, int64_t total, int max_ctx, int chunk,
-              int n_cu, float bytes_us) {
+struct PlanTime {
+    float us;
+    int64_t busy, grid;  // workgroups with work, and all
+    bool idle;           // some without
+};
+PlanTime plan_time(const DecodeCost &k, const int32_t *n_ctx, int n_seq, int streams, int64_t total, int max_ctx, int chunk,
+                   int n_cu, float bytes_us) {
+    PlanTime t;
     const int most = (max_ctx + chunk - 1) / chunk;
-    bool idle;
-    const int64_t busy = count_splits(n_ctx, n_seq, max_ctx, chunk, &idle) * streams;
-    const float cus = idle ? 0.875f : 1.0f;
+    t.busy = count_splits(n_ctx, n_seq, max_ctx, chunk, &t.idle) * streams;
+    t.grid = (int64_t)most * n_seq * streams;
+    const float cus = t.idle ? 0.875f : 1.0f;
     const float longest = k.fixed + k.round * ((std::min(chunk, max_ctx) + k.span - 1) / k.span);
-    float us = longest;
-    if (busy > cus * n_cu) {
-        const float work = busy * (k.fixed + 0.5f * k.round) + k.round * total * streams / k.span;
-        us = std::max(us, work / (cus * k.at_once) + 0.5f * longest);
+    t.us = longest;
+    if (t.busy > cus * n_cu) {
+        const float work = t.busy * (k.fixed + 0.5f * k.round) + k.round * total * streams / k.span;
+        t.us = std::max(t.us, work / (cus * k.at_once) + 0.5f * longest);
     }
-    return std::max(us, bytes_us + k.fixed) + (most > 1 ? kCombineUs : 0.0f);
+    t.us = std::max(t.us, bytes_us + k.fixed) + (most > 1 ? kCombineUs : 0.0f);
+    return t;
+}
+
+// Part of the even plan's estimate that a plan's has to stay below to take its place, 0 if it never
+// does (stored: the stored head dim; even_idle: the even plan has idle workgroups).  The estimate
+// knows little of how the dispatcher packs workgroups, so each kind of change has the margin with
+// which its shapes keep within the runs' noise of the even plan (3%, with a few at 5), measured over
+// 6000 shapes of 1 to 256 sequences of 60 to 32000 positions, equal and ragged.  (A margin of 2%
+// for all left 95 of the 1064 shapes that it changed 2 to 29% slower.)
+//   No split at all: 0.40 to 1.01 of the even plan's time, with less than 4% to gain up to 1.03.
+//   Never the 16x16 kernel in the place of an even plan on the integer one: a tenth more error against 64
+//     bits without a split, and with splits 0.83 to 1.21 of the time.
+//   Splits that leave workgroups idle in a grid of more than the CUs: integer ones on 256-dim rows
+//     0.41 to 0.92, on others up to 1.24; of the 16x16 kernel up to 1.20 beyond 5/8 of the CUs busy.
+//   Longer splits of the 16x16 kernel: 256-dim rows 0.55 to 0.80; 128-dim rows 0.75 to 1.06, mean 0.89;
+//     none on 64-dim rows (mean 0.97, up to 1.11).
+//   Integer splits in the place of the 16x16 kernel's: with one half of query heads, or 256-dim rows
+//     (with more halves on shorter rows 0.96 to 1.24); of fewer integer ones: 0.78 to 1.01, with less
+//     to gain up to 1.11; of none: with less than a quarter to gain up to 1.29.
+float plan_margin(const PlanTime &t, bool g4, bool split, const DecodePlan &even, bool even_idle, int G, int stored, int n_cu) {
+    if (even.g4 && !g4) return 0.0f;
+    if (!split) return even_idle ? 0.98f : 0.96f;
+    if (t.idle && t.grid > n_cu && (g4 ? stored < 256 : 8 * t.busy > 5 * n_cu)) return 0.0f;
+    if (!g4) return stored < 128 ? 0.0f : stored == 128 ? 0.8f : 0.98f;
+    if (!even.g4) return G <= 4 || stored == 256 ? 0.98f : 0.0f;
+    if (even.n_split == 1) return t.idle ? 0.0f : 0.75f;
+    return stored < 128 ? 0.8f : 0.9f;
 }
 }  // namespace
 
@@ -1516,7 +1549,8 @@ DecodePlan decode_plan_even(const int32_t *n_ctx, int n_seq, int n_kv, int G, in
 
 // Split plan: the kernel and the split length whose estimate is the lowest, among the batch's
 // context spread evenly (decode_plan_even) and equal shares of the longest sequence, fewest first;
-// a later one in that order has to gain 2%.  (The even plan alone gave a ragged batch of about as
+// a later one in that order has to gain 2%, and all of them the margin that their kind has over
+// the even plan (plan_margin).  (The even plan alone gave a ragged batch of about as
 // many streams as CUs a few second splits, which waited for the first ones, with a combine behind
 // them and idle workgroups between.  32 sequences of 700-1531 positions, 8 kv heads: 27.3 us with
 // two splits for some, 17.8 with none; 2000-6000: 36.4, 30.1; 64-dim rows, 1000-3000: 22.1, 13.2.
@@ -1554,14 +1588,16 @@ DecodePlan decode_plan(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_c
     const bool integer = G <= decode_int_gmax(stored_hd);
     const DecodeCost ki = int_cost(G, stored_hd, n_cu), kf = f16_cost(G, stored_hd, n_cu);
     auto time = [&](int chunk, bool g4) {
-        return plan_us(g4 ? ki : kf, n_ctx, n_seq, n_kv * (g4 ? 1 : groups), total, max_ctx, chunk, n_cu, bytes_us);
+        return plan_time(g4 ? ki : kf, n_ctx, n_seq, n_kv * (g4 ? 1 : groups), total, max_ctx, chunk, n_cu, bytes_us);
     };
+    const PlanTime even_t = time(even.chunk, even.g4);
     p = even;
-    float best = time(even.chunk, even.g4);
+    float best = even_t.us;
     auto weigh = [&](int chunk, bool g4) {
-        const float t = time(chunk, g4);
-        if (t < 0.98f * best) {
-            best = t;
+        const PlanTime t = time(chunk, g4);
+        if (t.us < 0.98f * best &&
+            t.us < plan_margin(t, g4, chunk < max_ctx, even, even_t.idle, G, stored_hd, n_cu) * even_t.us) {
+            best = t.us;
             p.g4 = g4;
             p.chunk = chunk;
         }
@@ -1574,9 +1610,7 @@ DecodePlan decode_plan(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_c
         // outlives the next tokens, as a captured one has to)
         const int chunk = ((max_ctx + k - 1) / k + (k > 1 ? 4 : 0) + 63) / 64 * 64;
         if (integer) weigh(chunk, true);
-        // (The 16x16 kernel never in the place of an even plan on the integer one: without splits a tenth
-        // more error against 64 bits, 3.3e-7 and 3.7e-7 over 28 to 75 sequences of 700 to 3000.)
-        if (!even.g4) weigh(chunk, false);
+        weigh(chunk, false);
     }
     p.n_split = (max_ctx + p.chunk - 1) / p.chunk;
     return p;
@@ -1693,9 +1727,8 @@ hipError_t launch_decode(const KvLayerView &L, int32_t *d_len, const int32_t *h_
     a.adv_len = adv && adv_in_kernel ? d_len : nullptr;
     a.adv_ctr = adv && adv_in_kernel ? adv : nullptr;
     dim3 grid(plan.n_split, L.H * a.NG, L.S);
-    // The integer kernel does less VALU work per window than the 16x16 one but has the longer
-    // per-window dependency chain; it runs when every wave streams at least 4 windows of its
-    // split (plan.g4).
+    // The integer kernel (plan.g4) does less VALU work per window than the 16x16 one but has the
+    // longer per-window dependency chain.
     const bool cap = softcap > 0.0f, norm = L.qn != nullptr || L.kn != nullptr;
     const bool pad = L.hdr != L.hd;
 #define TS_SPLIT(HDV, SC, NM)                                                                  \

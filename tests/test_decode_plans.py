@@ -44,6 +44,23 @@ def test_integer_kernel_keeps_unsplit_streams(n_seq, n_kv, G, ctx):
     assert plan(n_seq, n_kv, G, 64, ctx, ctx) == ("integer", 4, 1024, 1)
 
 
+@pytest.mark.parametrize("shape,want", [
+    ((16, 8, 4, 64, 3516, 3516), ("integer", 4, 3520, 1)),     # two integer splits for one: 15.2 us, 12.0
+    ((10, 8, 8, 64, 1629, 1629), ("integer", 4, 1664, 1)),
+    ((6, 2, 16, 128, 18562, 18562), ("integer", 4, 1088, 18)),
+    ((8, 8, 4, 64, 11833, 11833), ("integer", 4, 3968, 3)),
+    ((2, 8, 4, 128, 2, 7672), ("integer", 4, 704, 11)),        # not in a grid of idle workgroups: 16.0, 13.3
+    ((7, 8, 8, 128, 2091, 4182), ("16x16", 4, 384, 11)),       # 22.4, 20.0
+    ((6, 4, 12, 128, 2, 9471), ("16x16", 4, 512, 19)),         # 23.5, 20.3
+    ((24, 2, 6, 64, 2, 7583), ("16x16", 4, 384, 20)),          # 22.4, 18.3
+    ((3, 4, 12, 128, 10409, 10409), ("16x16", 4, 512, 21)),
+    ((1, 8, 4, 128, 801, 801), ("16x16", 4, 256, 4)),
+])
+def test_estimates_too_close_to_decide(shape, want):
+    """Shapes that an estimate a little lower had moved to a slower plan."""
+    assert plan(*shape) == want
+
+
 @pytest.mark.parametrize("shape", [(52, 8, 8, 128, 722, 1444), (43, 8, 5, 128, 1322, 1322), (20, 2, 16, 128, 4836, 4836),
                                    (2, 32, 1, 128, 2964, 2964), (14, 1, 8, 128, 15698, 15698)])
 def test_integer_kernel_is_not_replaced(shape):
