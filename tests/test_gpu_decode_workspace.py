@@ -8,6 +8,7 @@ import torch
 
 import airframe_amd
 from airframe_amd import _lib, synth
+from airframe_amd.kv_cache import decode_plan
 from tests.gpu_util import Pair, assert_close, dev, say
 from tests.test_gpu_decode import prefill_cache
 
@@ -63,6 +64,8 @@ def test_split_context_needs_a_workspace(gpu):
 @pytest.mark.parametrize("n_seq,n_kv,G,hd,lo,hi", [
     (16, 8, 4, 128, 4200, 4200),   # equal lengths: one split each, spread evenly
     (104, 16, 8, 256, 215, 264),   # one of 791 among them
+    (58, 2, 5, 256, 2376, 2376),   # one split each, spread evenly; the plan has two
+    (8, 32, 16, 256, 4071, 4135),  # ... with more partials than the library's scratch holds
 ])
 @pytest.mark.parametrize("fn", ["ts_attn_decode_append", "ts_attn_decode_append_noalloc"])
 def test_unsplit_context_needs_none(gpu, fn, n_seq, n_kv, G, hd, lo, hi):
@@ -70,6 +73,10 @@ def test_unsplit_context_needs_none(gpu, fn, n_seq, n_kv, G, hd, lo, hi):
     lens = np.linspace(lo, hi, n_seq).round().astype(int)
     if n_seq == 104:
         lens[0] = 791
+    n_cu = torch.cuda.get_device_properties(0).multi_processor_count
+    splits = decode_plan([int(n) + 1 for n in lens], n_kv, n_kv * G, hd, n_cu)["splits"]
+    assert n_cu != 256 or splits == (2 if n_seq in (58, 8) else 1)
+    assert n_seq != 8 or splits * n_seq * n_kv * G * (hd + 2) * 4 > 8 << 20
     rng, p = batch(n_seq, n_kv, hd, lens, n_seq)
     rc, out, ref = step(p, rng, n_kv, G, hd, fn)
     assert rc == _lib.TS_OK

@@ -63,9 +63,14 @@ def test_out_proj_tiles(gpu, n_tok, attn_dim, dim, planes):
     (weights.Q8_0, 70, 35, 512, 2, 1, 64),
     (weights.Q4_0, 33, 100, 256, 4, 2, 128),
     (weights.Q5_0, 70, 5, 512, 3, 1, 128),
+    (weights.Q4_K, 420, 1, 512, 64, 8, 64),    # decode rows: the last tile of 4 sequences
+    (weights.Q8_0, 550, 1, 256, 32, 8, 128),   # ... of half a tile's units
 ])
 def test_qkv_block_tiles(gpu, fmt, n_seq, n_tok, dim, n_head, n_kv, hd):
     say(f"qkv block tiles fmt={fmt} n_seq={n_seq} n_tok={n_tok} dim={dim} n_head={n_head} n_kv={n_kv} hd={hd}")
+    # (more than 256 tiles of 32 rows x 256 columns: the tile kernel takes them)
+    rows32 = -(-n_seq // 32) if n_tok == 1 else n_seq * (n_tok // 32 + 2)
+    assert rows32 * (-(-n_head * hd // 256) + -(-n_kv * hd // 128)) > 256
     rng = np.random.default_rng(fmt + dim + n_tok)
     p = Pair(n_seq, n_kv, hd, 100 + n_tok, 1e6)
     p.set_lens(rng.integers(0, 97, size=n_seq).astype(np.int32))
@@ -86,12 +91,45 @@ def test_qkv_block_tiles(gpu, fmt, n_seq, n_tok, dim, n_head, n_kv, hd):
     p.check_codes()
 
 
+@pytest.mark.parametrize("fmt,n_seq,n_tok,hd", [(weights.Q4_K, 70, 35, 64), (weights.Q5_0, 70, 35, 128), (weights.Q8_0, 550, 1, 128)])
+def test_qkv_block_tiles_norm(gpu, fmt, n_seq, n_tok, hd):
+    """With the QK norm; and without the raw K and V: the same q and cache bits."""
+    say(f"qkv block tiles with norm fmt={fmt} n_seq={n_seq} n_tok={n_tok} hd={hd}")
+    rng = np.random.default_rng(fmt + hd)
+    dim, n_kv = 256, 2 if n_tok > 1 else 8
+    n_head = 2 * n_kv
+    lens = rng.integers(0, 97, size=n_seq).astype(np.int32)
+    norms = [(rng.standard_normal(hd) * 0.4 + 1.0).astype(np.float32) for _ in range(2)]
+    w = [dev(random_blob(rng, fmt, r * hd, dim)) for r in (n_head, n_kv, n_kv)]
+    x = dev(rng.standard_normal((n_seq, n_tok, dim)).astype(np.float32))
+    caches = [Pair(n_seq, n_kv, hd, 100 + n_tok, 1e6) for _ in range(2)]
+    for p in caches:
+        p.set_lens(lens)
+        p.gpu.set_qk_norm(0, dev(norms[0]), dev(norms[1]), 1e-6)
+    k_out = torch.empty((n_seq, n_tok, n_kv, hd), dtype=torch.float32, device="cuda")
+    v_out = torch.empty_like(k_out)
+    q = caches[0].gpu.qkv_append_gguf(0, x, fmt, *w, caches[0].rope, kv_out=(k_out, v_out))
+    q2 = caches[1].gpu.qkv_append_gguf(0, x, fmt, *w, caches[1].rope)
+    torch.cuda.synchronize()
+    assert torch.equal(q, q2)
+    ora = caches[0].ora
+    ora.q_norm, ora.k_norm, ora.norm_eps = norms[0], norms[1], 1e-6
+    ora.append(k_out.cpu().numpy(), v_out.cpu().numpy())
+    caches[1].ora = ora
+    for p in caches:
+        p.gpu.increment(n_tok)
+    ora.advance(n_tok)
+    for p in caches:
+        p.check_codes()
+
+
 @pytest.mark.parametrize("fmt,n_tok,attn_dim,dim", [
-    (weights.Q4_K, 900, 256, 2049), (weights.Q5_K, 8195, 256, 8), (weights.Q8_0, 830, 512, 1800),
-    (weights.Q4_0, 900, 768, 2300), (weights.Q5_0, 641, 256, 2560),
+    (weights.Q4_K, 900, 256, 2049), (weights.Q5_K, 8195, 256, 8), (weights.Q8_0, 1030, 512, 1800),
+    (weights.Q4_0, 900, 768, 2300), (weights.Q5_0, 830, 256, 2500),
 ])
 def test_out_proj_block_tiles(gpu, fmt, n_tok, attn_dim, dim):
     say(f"out_proj block tiles fmt={fmt} n_tok={n_tok} attn_dim={attn_dim} dim={dim}")
+    assert -(-n_tok // 32) * -(-dim // 256) > 256  # the tile kernel takes them
     rng = np.random.default_rng(fmt + n_tok + dim)
     blob = random_blob(rng, fmt, dim, attn_dim)
     a = rng.standard_normal((n_tok, attn_dim)).astype(np.float32)

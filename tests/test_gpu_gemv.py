@@ -15,35 +15,37 @@ from tests.test_gpu_weights import random_blob
 
 pytestmark = pytest.mark.gpu
 
-FORMS = [1, 2, weights.Q4_K, weights.Q5_K, weights.Q8_0, weights.Q4_0, weights.Q5_0]  # 1, 2: f16 planes
+PLANES = {"f16": 1, "f16x2": 2}
+BLOCKS = {"q4_k": weights.Q4_K, "q5_k": weights.Q5_K, "q8_0": weights.Q8_0, "q4_0": weights.Q4_0, "q5_0": weights.Q5_0}
+FORMS = [*PLANES, *BLOCKS]
 
 
 def matrix(rng, form, rows, cols):
     """(device tensor, f32 values) of a weight matrix."""
-    if form in (1, 2):
+    if form in PLANES:
         w = (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32)
         hi = w.astype(np.float16)
-        if form == 1:
+        if form == "f16":
             return dev(hi), hi.astype(np.float32)
         lo = (w - hi.astype(np.float32)).astype(np.float16)
         return dev(np.concatenate([hi, lo], 1)), hi.astype(np.float32) + lo.astype(np.float32)
-    blob = random_blob(rng, form, rows, cols)
-    return dev(blob), oracle.dequant(form, blob, rows * cols).reshape(rows, cols)
+    blob = random_blob(rng, BLOCKS[form], rows, cols)
+    return dev(blob), oracle.dequant(BLOCKS[form], blob, rows * cols).reshape(rows, cols)
 
 
 @pytest.mark.parametrize("form", FORMS)
 @pytest.mark.parametrize("n_tok,attn_dim,dim", [(1, 256, 9), (1, 1280, 200), (2, 512, 33), (1, 8448, 24), (2, 8448, 17)])
 def test_out_proj_rows(gpu, form, n_tok, attn_dim, dim):
     say(f"out_proj rows form={form} n_tok={n_tok} attn_dim={attn_dim} dim={dim}")
-    rng = np.random.default_rng(form * 7 + attn_dim + dim)
+    rng = np.random.default_rng(FORMS.index(form) * 7 + attn_dim + dim)
     w, wf = matrix(rng, form, dim, attn_dim)
     a = rng.standard_normal((n_tok, attn_dim)).astype(np.float32)
     act = (rng.standard_normal((n_tok, dim)) * 4).astype(np.float32)
     act_d, stash_d = dev(act), torch.zeros((n_tok, dim), dtype=torch.float32, device="cuda")
-    if form in (1, 2):
-        attn_out_proj(dev(a), w, act_d, stash=stash_d, planes=form)
+    if form in PLANES:
+        attn_out_proj(dev(a), w, act_d, stash=stash_d, planes=PLANES[form])
     else:
-        attn_out_proj_gguf(dev(a), form, w, dim, act_d, stash=stash_d)
+        attn_out_proj_gguf(dev(a), BLOCKS[form], w, dim, act_d, stash=stash_d)
     torch.cuda.synchronize()
     dot = oracle.project_f32(a, wf)
     assert_close(stash_d.cpu().numpy(), dot, "projection")
@@ -54,7 +56,7 @@ def test_out_proj_rows(gpu, form, n_tok, attn_dim, dim):
 @pytest.mark.parametrize("n_seq,dim,n_head,n_kv,hd", [(1, 768, 3, 1, 128), (2, 1280, 4, 2, 64), (1, 512, 2, 1, 96)])
 def test_qkv_rows(gpu, form, n_seq, dim, n_head, n_kv, hd):
     say(f"qkv rows form={form} n_seq={n_seq} dim={dim} n_head={n_head} n_kv={n_kv} hd={hd}")
-    rng = np.random.default_rng(form * 11 + dim)
+    rng = np.random.default_rng(FORMS.index(form) * 11 + dim)
     p = Pair(n_seq, n_kv, hd, 70, 1e6)
     for start in (0, 31, 62):  # the first, the last and a middle position of a V block
         p.set_lens(np.full(n_seq, start, np.int32))
@@ -63,12 +65,12 @@ def test_qkv_rows(gpu, form, n_seq, dim, n_head, n_kv, hd):
         k_out = torch.empty((n_seq, 1, n_kv, hd), dtype=torch.float32, device="cuda")
         v_out = torch.empty_like(k_out)
         args = (wq, wk, wv, p.rope)
-        if form in (1, 2):
-            q = p.gpu.qkv_append(0, dev(x), *args, kv_out=(k_out, v_out), planes=form)
-            q2 = p.gpu.qkv_append(0, dev(x), *args, planes=form)  # K and V through the workspace
+        if form in PLANES:
+            q = p.gpu.qkv_append(0, dev(x), *args, kv_out=(k_out, v_out), planes=PLANES[form])
+            q2 = p.gpu.qkv_append(0, dev(x), *args, planes=PLANES[form])  # K and V through the workspace
         else:
-            q = p.gpu.qkv_append_gguf(0, dev(x), form, *args, kv_out=(k_out, v_out))
-            q2 = p.gpu.qkv_append_gguf(0, dev(x), form, *args)
+            q = p.gpu.qkv_append_gguf(0, dev(x), BLOCKS[form], *args, kv_out=(k_out, v_out))
+            q2 = p.gpu.qkv_append_gguf(0, dev(x), BLOCKS[form], *args)
         torch.cuda.synchronize()
         assert torch.equal(q, q2)
         q, k_out, v_out = q.cpu().numpy(), k_out.cpu().numpy(), v_out.cpu().numpy()
