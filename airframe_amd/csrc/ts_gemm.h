@@ -76,8 +76,10 @@ constexpr int kValu = 2, kMfma = 8, kVmemRead = 0x20, kDsRead = 0x100, kDsWrite 
 // 2048 x 2560, 4096 long: 199, 149 (all CUs together reach about 1.1 PFLOP/s on f16 matrix
 // instructions; chunks of 32 k in a row took 164 and 134, but add in another order, and a last bit
 // moves a key or value next to a code's edge).
-// LDS bounds it: per chunk 48 KB read at 128 and 24 KB written at 75 bytes a clock, ~710 clocks
-// against 512 of matrix work.  128-row tiles (8 waves, or 4 of 64 x 128) were slower.
+// Its loads bound it (counters, 2048 x 6144): of the CUs' busy cycles the address path works 91%, ~50
+// cycles for a load of 1 KB, the matrix cores 39% and LDS 30%.  A chunk takes two 32-byte pieces of
+// a weight row's 128-byte line and the next chunk the other two, a step later.  128-row tiles (8
+// waves, or 4 of 64 x 128) were slower.
 __device__ __forceinline__ void gemm_tile_core(GemmTiles &sm, const float *xs, const _Float16 *const (&ws)[4],
                                                int nch, int xwrap, int tid, floatx16 (&acc)[2][2]) {
     const int wave = tid >> 6, lane = tid & 63, j = lane & 31, hf = lane >> 5;

@@ -566,8 +566,10 @@ __device__ inline float kq_quad_sum(float v) {
 // 32 rb + .., columns 32 w + .. in acc[rb].  A block decoded once serves 64 rows here against 32
 // in the slice loops above, which spend twice as long on decoding (VALU) as on matrix
 // instructions: 2000 tokens, a block of 4096-wide projections, Q4_K 752 -> 551 us, Q5_K 849 -> 572,
-// Q8_0 1159 -> 589, Q4_0 939 -> 570, Q5_0 1401 -> 631.  LDS bounds it (every wave reads all x operands: 128 KB a
-// chunk at 128 bytes a clock, as long as the chunk's matrix work).  Eight waves of one weight row per lane rather than four of two: the latter
+// Q8_0 1159 -> 589, Q4_0 939 -> 570, Q5_0 1401 -> 631.  No single
+// unit bounds it (counters, Q4_K, 2048 x 6144): of the CUs' busy cycles address path and matrix cores work 43%
+// each and LDS 29%; a wave's block decode and matrix work are one chain between barriers.
+// Eight waves of one weight row per lane rather than four of two: the latter
 // spill at two waves per SIMD, and a spilled register waits for every load in flight.
 // x goes through LDS in chunks of 64 k, one barrier a chunk; the block bytes of a lane's weight
 // row (wb, at super-block 0) are loaded straight into its registers L chunks ahead.  xs: the

@@ -119,7 +119,8 @@ __global__ __launch_bounds__(256) void proj_split_kernel(ProjArgs p) {
 }
 
 // The same with the weights as GGUF K-quant blocks read in the loop (gemm_split_kq); slices of
-// whole super-blocks, one slice when the tiles alone fill the chip.
+// whole super-blocks, one slice where 256 tiles or more do not take the tile kernel (kq_tiles, or an
+// output that shares memory with the input).
 template <int T>
 __global__ __launch_bounds__(256) void proj_split_kq_kernel(ProjArgs p) {
     __shared__ __align__(16) KqTiles sm[2];

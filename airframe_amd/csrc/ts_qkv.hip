@@ -454,8 +454,9 @@ __global__ __launch_bounds__(256) void qkv_split_kernel(QkvArgs a) {
 }
 
 // The same with the weights as GGUF K-quant blocks read in the loop (gemm_split_kq); a slice
-// is a whole number of 256-element super-blocks.  Also used with one slice (no split) for
-// shapes with many tiles, the reduce kernel then only running the epilogue.
+// is a whole number of 256-element super-blocks.  One slice (no split), the reduce kernel then only
+// running the epilogue, where 256 tiles or more do not take the tile kernel (kq_tiles, or an output
+// that shares memory with x).
 template <int T>
 __global__ __launch_bounds__(256) void qkv_split_kq_kernel(QkvArgs a) {
     __shared__ __align__(16) KqTiles sm[2];
