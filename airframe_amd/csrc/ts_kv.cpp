@@ -489,19 +489,18 @@ static int attn_decode(const ts_kv *kv, int32_t layer, const float *d_q, int32_t
                                           kv->n_cu, kv->hdp, k_new != nullptr);
     // partials [S][n_head][n_split][hd], then m and l [S][n_head][n_split]
     const uint64_t per_split = (uint64_t)kv->d.n_seq * n_head * (kv->hdp + 2) * sizeof(float);
-    uint64_t need = plan.n_split * per_split;
-    // a caller's: plan.n_split <= decode_cap(max_seq), the count the workspace was sized for
+    // Which calls have to have room for partials does not change with the plan that is taken in the end:
+    // those whose evenly spread context is split, for its splits (library's scratch) or for any
+    // (a caller's workspace; plan.n_split <= decode_cap(max_seq), the count it was sized for).
+    uint64_t need = plan.even_split * per_split;
     if (!noalloc) ts_attn_decode_workspace(kv, n_head, &need);
     const int rc_ws = !d_workspace || workspace_bytes < need ? TS_ERR_WORKSPACE
                       : !aligned16(d_workspace)              ? TS_ERR_INVALID
                                                              : TS_OK;
-    // Which calls of a caller have to bring a workspace does not change with the plan that is taken
-    // in the end.
-    if (!noalloc && plan.even_split > 1 && rc_ws != TS_OK) return rc_ws;
-    if (plan.n_split > 1 && rc_ws != TS_OK) {
+    if (plan.even_split > 1 && rc_ws != TS_OK) return rc_ws;
+    // A plan with more partials than there is room for gives way to the even one.
+    if (plan.n_split > 1 && (rc_ws != TS_OK || plan.n_split * per_split > workspace_bytes))
         plan = ts::decode_plan_even(ctx.data(), kv->d.n_seq, kv->d.n_head_kv, n_head / kv->d.n_head_kv, kv->n_cu, kv->hdp);
-        if (plan.n_split > 1 && (!noalloc || plan.n_split * per_split > workspace_bytes)) return rc_ws;
-    }
     // An eager call takes the host's lengths as launch arguments (the device's agree with them
     // unless a captured call changed them); one being captured reads the device lengths, so
     // that replays see the lengths of their time.

@@ -235,10 +235,11 @@ int ts_attn_decode_append(ts_kv *kv, int32_t layer, const float *d_k, const floa
  * split partials go to a scratch array the library keeps on every GPU it runs on (8 MiB each,
  * until the process ends).  No counterpart in the reference: for callers that cannot allocate
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
- * Returns TS_ERR_WORKSPACE when this call's partials, n_seq * n_head * splits * (hds + 2)
- * floats, would exceed 8 MiB, where hds is the stored head dim: head_dim rounded up to 64,
- * 128 or 256 (a call that needs no split needs none).  All calls on one GPU
- * share the array: calls that overlap on one GPU (other streams, other threads) race. */
+ * Returns TS_ERR_WORKSPACE when the partials of the call's context, spread evenly over the
+ * compute units, n_seq * n_head * splits * (hds + 2) floats, would exceed 8 MiB, where hds is the
+ * stored head dim: head_dim rounded up to 64, 128 or 256 (a context that is not split so needs
+ * none).  All calls on one GPU share the array: calls that overlap on one GPU (other streams,
+ * other threads) race. */
 int ts_attn_decode_append_noalloc(ts_kv *kv, int32_t layer, const float *d_k, const float *d_v,
                                   const float *d_q, int32_t n_head, const ts_rope *rope, float softcap,
                                   float *d_out, void *stream);

@@ -61,6 +61,21 @@ def test_split_context_needs_a_workspace(gpu):
     assert_close(out, ref, "with a workspace")
 
 
+def test_split_context_beyond_the_scratch(gpu):
+    """... and refused without allocation where its partials exceed the library's scratch, whatever plan
+    a caller's workspace gets."""
+    say("noalloc decode beyond the scratch: refused")
+    lens = np.linspace(150, 301, 65).astype(int)
+    n_cu = torch.cuda.get_device_properties(0).multi_processor_count
+    assert n_cu != 256 or decode_plan([int(n) + 1 for n in lens], 8, 64, 256, n_cu)["splits"] == 1
+    rng, p = batch(65, 8, 256, lens, 2)
+    assert step(p, rng, 8, 8, 256, "ts_attn_decode_append_noalloc")[0] == _lib.TS_ERR_WORKSPACE
+    ws = p.gpu.workspace(64)
+    rc, out, ref = step(p, rng, 8, 8, 256, "ts_attn_decode_append", ws.data_ptr(), ws.numel())
+    assert rc == _lib.TS_OK
+    assert_close(out, ref, "with a workspace")
+
+
 @pytest.mark.parametrize("n_seq,n_kv,G,hd,lo,hi", [
     (16, 8, 4, 128, 4200, 4200),   # equal lengths: one split each, spread evenly
     (104, 16, 8, 256, 215, 264),   # one of 791 among them
