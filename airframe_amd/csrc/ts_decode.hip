@@ -1396,6 +1396,7 @@ windows_done:
 
 namespace {
 constexpr int kMinChunk = 256;  // splits shorter than this leave waves without a window
+constexpr int kIntChunk = 1024;  // the shortest evenly spread splits that take the integer kernel
 
 // Splits of `chunk` positions of all sequences; *idle: some sequence has fewer than the longest, whose
 // grid then holds workgroups without work.
@@ -1524,7 +1525,7 @@ static DecodePlan even_plan(const int32_t *n_ctx, int n_seq, int n_kv, int G, in
     p.g4 = false;
     if (G <= decode_int_gmax(stored_hd)) {
         p.chunk = even_chunk(n_ctx, n_seq, n_kv, n_cu - n_cu / 8, total, max_ctx);
-        p.g4 = p.chunk >= 1024;
+        p.g4 = p.chunk >= kIntChunk;
     }
     if (!p.g4) p.chunk = even_chunk(n_ctx, n_seq, n_kv * ((G + 7) / 8), 2 * n_cu, total, max_ctx);
     p.n_split = p.even_split = (max_ctx + p.chunk - 1) / p.chunk;
@@ -1573,11 +1574,14 @@ DecodePlan decode_plan(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_c
     // one window per wave does not pay: 8.5 windows per wave took 26.6 us per layer on config 2's
     // shape against 10.0 with splits and a combine.
     // (Not in the place of the integer kernel without a split, which serves about as many streams as
-    // CUs: 256 streams of 1000 64-dim positions 9.8 us a layer, 12.6 with 16 waves.)
-    const DecodePlan even = even_plan(n_ctx, n_seq, n_kv, G, n_cu, stored_hd, total, max_ctx);
+    // CUs: 256 streams of 1000 64-dim positions 9.8 us a layer, 12.6 with 16 waves.  Shorter contexts
+    // need no even plan to know.)
+    auto integer_even = [&] {
+        return (max_ctx + 63) / 64 * 64 >= kIntChunk && even_plan(n_ctx, n_seq, n_kv, G, n_cu, stored_hd, total, max_ctx).g4;
+    };
     const int n_win = (max_ctx - (fused ? 1 : 0) + 63) / 64;
     const int wmax = stored_hd <= 64 ? 16 : stored_hd <= 128 ? 8 : 4;
-    if (!even.g4 && n_win > 4 && n_win <= wmax && (int64_t)n_seq * n_kv * groups <= n_cu) {
+    if (n_win > 4 && n_win <= wmax && (int64_t)n_seq * n_kv * groups <= n_cu && !integer_even()) {
         p.g4 = false;
         p.nw = n_win <= 8 ? 8 : 16;
         p.chunk = (max_ctx + 63) / 64 * 64;
@@ -1587,6 +1591,7 @@ DecodePlan decode_plan(const int32_t *n_ctx, int n_seq, int n_kv, int G, int n_c
     const float bytes_us = (float)total * n_kv * (stored_hd + 8) / kDecodeBytesUs;
     const bool integer = G <= decode_int_gmax(stored_hd);
     const DecodeCost ki = int_cost(G, stored_hd, n_cu), kf = f16_cost(G, stored_hd, n_cu);
+    const DecodePlan even = even_plan(n_ctx, n_seq, n_kv, G, n_cu, stored_hd, total, max_ctx);
     auto time = [&](int chunk, bool g4) {
         return plan_time(g4 ? ki : kf, n_ctx, n_seq, n_kv * (g4 ? 1 : groups), total, max_ctx, chunk, n_cu, bytes_us);
     };
